@@ -13,7 +13,7 @@ LIB = os.path.join(HERE, "libdkt.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("DKT_OFFLOAD_ARCH", "gfx950")
 
-HOST_SRCS = ["mesh.cpp", "capi_mesh.cpp"]
+HOST_SRCS = ["mesh.cpp", "capi_mesh.cpp", "point_plan.cpp"]
 HIP_SRCS = ["plan.hip", "cg.hip", "batch.hip"]
 
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-fopenmp", "-ffp-contract=off", "-Wall", "-Wno-unused-variable",

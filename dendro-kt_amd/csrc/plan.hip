@@ -33,6 +33,7 @@
 #include "plan_impl.h"
 #include "tile_kernel.h"
 #include "conf_kernel.h"
+#include "point_kernel.h"
 
 namespace dkt {
 const MeshParams &da_params(const dkt_da *da);
@@ -892,6 +893,48 @@ void build_tiled(dkt_plan *pl, const MeshParams &mp, const Traversal &tr, int re
 }
 
 // ---------------------------------------------------------------------------
+// Point tiles (p = 1; point_plan.h).
+// ---------------------------------------------------------------------------
+template <typename T>
+size_t point_lds(const dkt_plan *pl) {
+  return point_lds_bytes<T>(pl->max_slots, pl->max_units, pl->max_grp * pl->npe);
+}
+
+void upload_points(dkt_plan *pl, PointHost &o, int T) {
+  pl->points = true;
+  pl->tile_leaves = T;
+  pl->ntiles = o.tiles.size();
+  pl->nshared = o.snode.size();
+  pl->npartial = o.npartial;
+  pl->max_nodes = o.max_nodes;
+  pl->max_hang = o.max_hang;
+  pl->stats = o.stats;
+  pl->map_bytes = (double)o.bytes();
+  pl->ptiles.upload(nonempty(std::move(o.tiles)));
+  pl->tile_blocks.upload(nonempty(std::move(o.blocks)));
+  pl->leaf_loc.upload(nonempty(std::move(o.lloc)));
+  pl->leaf_aux.upload(nonempty(std::move(o.laux)));
+  pl->snode.upload(nonempty(std::move(o.snode)));
+  pl->soff.upload(o.soff);
+}
+
+// Leaves per tile: the requested size, else kPointTile, halved until the LDS
+// footprint (FP64) fits.
+void build_points(dkt_plan *pl, const MeshParams &mp, const Traversal &tr, int requested) {
+  int T = requested ? requested : kPointTile;
+  while (true) {
+    PointHost o = build_points_reference(mp, tr, pl->N, T, std::max(1, T / pl->npe));
+    pl->max_slots = o.max_slots + (o.max_slots & 1);
+    pl->max_units = o.max_units;
+    pl->max_grp = o.max_grp;
+    pl->lds_bytes = point_lds<double>(pl);
+    if (pl->lds_bytes <= kLdsLimit) return upload_points(pl, o, T);
+    if (requested || T <= 64) throw std::runtime_error("tile does not fit in LDS");
+    T /= 2;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Tiled conforming operator construction (conf_kernel.h).
 // ---------------------------------------------------------------------------
 void build_conf_tiled(dkt_plan *pl, const MeshParams &mp, const Traversal &tr, int T) {
@@ -1298,6 +1341,39 @@ void run_tiled(dkt_plan *pl, int nrhs, const T *x, T *y, int mask, hipStream_t s
   }
 }
 
+// Columns of one launch over point tiles: kPointCols, which bounds the partial
+// sums (a column's tiles run next to each other, so more columns in a launch
+// gain nothing), or as many as fit in the caller's scratch.
+constexpr int kPointCols = 8;
+
+template <typename T, int DIM>
+void run_points(dkt_plan *pl, int nrhs, const T *x, T *y, int mask, hipStream_t st, const int *cancel,
+                const ExtScratch *ext) {
+  const bool f64 = sizeof(T) == 8;
+  const T *kmat = f64 ? (const T *)pl->kmat64.p : (const T *)pl->kmat32.p;
+  int chunk = std::min(nrhs, kPointCols);
+  while (ext && chunk > 1 && pl->npartial * (size_t)chunk * sizeof(T) > ext->bytes) chunk--;
+  T *part = matvec_scratch<T>(pl, std::max<size_t>(1, pl->npartial * (size_t)chunk), ext);
+  for (int q0 = 0; q0 < nrhs; q0 += chunk) {
+    const int nq = std::min(chunk, nrhs - q0);
+    const PtArgs A = pl->point_args(mask, cancel, nq, nrhs);
+    if (pl->ntiles * (size_t)nq > (size_t)INT32_MAX) throw std::invalid_argument("too many tiles and columns");
+    if (pl->profiling && !ext) HIP_OK(hipEventRecord(pl->next_event(), st));
+    if (pl->ntiles) {
+      hipLaunchKernelGGL((point_kernel<T, DIM, false>), dim3(pl->ntiles * nq), dim3(pl->tile_leaves),
+                         point_lds<T>(pl), st, A, kmat, x + q0, y + q0, part);
+      HIP_OK(hipGetLastError());
+    }
+    if (pl->profiling && !ext) HIP_OK(hipEventRecord(pl->next_event(), st));
+    if (pl->nshared) {
+      hipLaunchKernelGGL((fixup_kernel<T>), dim3((pl->nshared + 255) / 256), dim3(256), 0, st, (int)pl->nshared,
+                         pl->snode.p, pl->soff.p, part, A.dir_out, nq, nrhs, y + q0, cancel);
+      HIP_OK(hipGetLastError());
+    }
+    if (pl->profiling && !ext) HIP_OK(hipEventRecord(pl->next_event(), st));
+  }
+}
+
 template <typename T, int DIM, int P>
 void run_conf(dkt_plan *pl, int nrhs, const T *x, T *y, int mask, hipStream_t st, const int *cancel,
               const ExtScratch *ext) {
@@ -1363,6 +1439,8 @@ void run_matvec(dkt_plan *pl, int nrhs, const T *x, T *y, int mask, hipStream_t 
       run_simple<T, D, P>(pl, nrhs, x, y, mask, st, cancel, ext);  \
     else if (pl->conforming)                                       \
       run_conf<T, D, P>(pl, nrhs, x, y, mask, st, cancel, ext);    \
+    else if constexpr (point_tiles(D, P))                          \
+      run_points<T, D>(pl, nrhs, x, y, mask, st, cancel, ext);     \
     else                                                           \
       run_tiled<T, D, P>(pl, nrhs, x, y, mask, st, cancel, ext);   \
     return;                                                        \
@@ -1445,6 +1523,8 @@ extern "C" int dkt_plan_create(const dkt_da *da, int op, const double *op_data, 
       build_simple(pl.get(), mp, tr);
     else if (pl->conforming)
       build_conf_tiled(pl.get(), mp, tr, tshift ? 1 << tshift : 256);
+    else if (point_tiles(mp.dim, mp.order))
+      build_points(pl.get(), mp, tr, tshift ? 1 << tshift : 0);
     else
       build_tiled(pl.get(), mp, tr, tshift ? 1 << tshift : 0);
     *out = pl.release();

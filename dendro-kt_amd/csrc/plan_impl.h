@@ -7,6 +7,7 @@
 #include "../../include/dkt.h"
 #include "plan_common.h"
 #include "conf_kernel.h"
+#include "point_kernel.h"
 
 // Solver workspace: CG vectors and reduction partials, allocated on first use.
 struct CgWorkspace {
@@ -59,6 +60,16 @@ struct dkt_plan {
   dkt::DevBuf<uint32_t> leaf_aux, carry_key;
   dkt::DevBuf<uint32_t> hentries;
   dkt::DevBuf<uint64_t> blocks;
+  // point tiles (p = 1)
+  bool points = false;
+  int max_slots = 0, max_units = 0;
+  dkt::DevBuf<dkt::PtTile> ptiles;
+  dkt::DevBuf<uint32_t> tile_blocks;
+  // The kernel arguments of a matvec over the point tiles.
+  dkt::PtArgs point_args(int mask, const int *cancel, int nq, int ld) const {
+    return dkt::PtArgs{ptiles.p,  tile_blocks.p, leaf_loc.p, leaf_aux.p, mask == 1 ? dirichlet.p : nullptr,
+                       mask ? dirichlet.p : nullptr, cancel, op, hp, nq, ld, max_slots, max_units};
+  }
   // conforming tiles
   dkt::DevBuf<dkt::ConfTileHdr> ctiles;
   dkt::DevBuf<uint16_t> virt_off;
