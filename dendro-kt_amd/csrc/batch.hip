@@ -221,20 +221,20 @@ struct PointBatchPlan {
 };
 
 // All tiles and columns of a batch of point plans of one dim in one launch.
-template <typename T, int DIM>
+template <typename T, int DIM, bool CAP>
 __global__ void __launch_bounds__(kTileThreads) point_kernel_batch(const PointBatchPlan<T> *__restrict__ plans,
                                                                    const int *__restrict__ item_start, int nplans) {
   const int t = xcd_tile(blockIdx.x, gridDim.x);
   const int k = find_range(item_start, nplans, t);
   const PointBatchPlan<T> bp = plans[k];  // a copy: its fields live in scalar registers
   if (bp.A.cancel && *bp.A.cancel) return;
-  point_body<T, DIM, false>(bp.A, t - item_start[k], bp.kref, bp.x, bp.y, bp.partial);
+  point_body<T, DIM, CAP>(bp.A, t - item_start[k], bp.kref, bp.x, bp.y, bp.partial);
 }
 
 // Point plans of one dim: one tile launch with one record per (column chunk,
 // plan).  A chunk's columns are separate work items of the launch; column-major
 // vectors take one record per column.
-template <typename T, int DIM>
+template <typename T, int DIM, bool CAP>
 struct PointGroup : GroupBase, FixSource<T> {
   GroupMem mem;
   PointBatchPlan<T> *table = nullptr;
@@ -283,7 +283,7 @@ struct PointGroup : GroupBase, FixSource<T> {
 
   void launch(hipStream_t st) override {
     if (nitems)
-      hipLaunchKernelGGL((point_kernel_batch<T, DIM>), dim3(nitems), dim3(threads), lds, st, table, item_start, nrec);
+      hipLaunchKernelGGL((point_kernel_batch<T, DIM, CAP>), dim3(nitems), dim3(threads), lds, st, table, item_start, nrec);
     HIP_OK(hipGetLastError());
   }
 };
@@ -400,8 +400,8 @@ struct ConfGroup : GroupBase, FixSource<T> {
 };
 
 template <typename T>
-// kind: 0 reference-semantics tiles, 1 conforming tiles, 2 conforming tiles
-// with per-level captured element matrices.
+// kind: 0 reference-semantics tiles, 1 conforming tiles, 3 point tiles; 2 and 4
+// those of 1 and 3 with per-level captured element matrices.
 GroupBase *make_group(int kind, int dim, int p, const std::vector<dkt_plan *> &pls,
                       const std::vector<const void *> &xs, const std::vector<void *> &ys, int nrhs, int masked,
                       const std::vector<const int *> &cancel = {}, DevArena *arena = nullptr, int max_cols = 0,
@@ -412,9 +412,13 @@ GroupBase *make_group(int kind, int dim, int p, const std::vector<dkt_plan *> &p
       return new ConfGroup<T, D, PP, true>(pls, xs, ys, nrhs, masked, cancel, arena, max_cols, colmajor);    \
     if (kind == 1)                                                                                           \
       return new ConfGroup<T, D, PP, false>(pls, xs, ys, nrhs, masked, cancel, arena, max_cols, colmajor);   \
-    if constexpr (point_tiles(D, PP))                                                                        \
-      return new PointGroup<T, D>(pls, xs, ys, nrhs, masked, cancel, arena, max_cols, colmajor);             \
-    else                                                                                                     \
+    if constexpr (PP == 1) {                                                                                 \
+      if (kind == 3)                                                                                         \
+        return new PointGroup<T, D, false>(pls, xs, ys, nrhs, masked, cancel, arena, max_cols, colmajor);    \
+      if (kind == 4)                                                                                         \
+        return new PointGroup<T, D, true>(pls, xs, ys, nrhs, masked, cancel, arena, max_cols, colmajor);     \
+    }                                                                                                        \
+    if constexpr (!point_tiles(D, PP))                                                                       \
       return new Group<T, D, PP>(pls, xs, ys, nrhs, masked, cancel, arena, max_cols, colmajor);              \
   }
   DKT_GROUP(2, 1)
@@ -433,7 +437,7 @@ std::map<std::tuple<int, int, int>, std::vector<int>> by_kind_of(dkt_plan *const
     dkt_plan *pl = plans[k];
     if (pl->dry || pl->simple || (pl->per_level && !pl->conforming))
       throw std::invalid_argument("batch plans must be tiled device plans (reference or conforming)");
-    by_kind[{pl->conforming ? (pl->per_level ? 2 : 1) : 0, pl->dim, pl->order}].push_back(k);
+    by_kind[{(pl->points ? 3 : pl->conforming ? 1 : 0) + (pl->per_level ? 1 : 0), pl->dim, pl->order}].push_back(k);
   }
   return by_kind;
 }

@@ -131,11 +131,16 @@ struct Renumber {
   uint16_t operator()(int32_t ref) const { return ref >= 0 ? node[ref] : point[-1 - ref]; }
 };
 
+// A tile that does not fit the layout.
+struct Misfit : std::runtime_error {
+  using std::runtime_error::runtime_error;
+};
+
 // Orders a tile's nodes and points and writes its rows and sums.  In: nodes by
 // first touch, the points, corr: the node of each correction slot.
 void finish_tile(TileOut &to, PointSet &ps, const std::vector<uint16_t> &corr, Renumber &rn) {
   const size_t nn = to.nodes.size(), np = ps.pts.size(), nc = corr.size();
-  if (nn + np + nc + 1 > (size_t)kPtMaxPoints) throw std::runtime_error("tile has too many points");
+  if (nn + np + nc + 1 > (size_t)kPtMaxPoints) throw Misfit("tile has too many points");
   // Levels: a row's level is one more than its higher end's (ends come first).
   std::vector<uint8_t> lev(np, 0);
   int nlev = 0;
@@ -146,7 +151,7 @@ void finish_tile(TileOut &to, PointSet &ps, const std::vector<uint16_t> &corr, R
     lev[i] = (uint8_t)(1 + std::max(la, lb));
     nlev = std::max(nlev, (int)lev[i]);
   }
-  if (nlev > kPtLevels) throw std::runtime_error("tile has too many row levels");
+  if (nlev > kPtLevels) throw Misfit("tile has too many row levels");
   for (size_t i = np; i-- > 0;) {  // the ends of a live row are live
     const Point &p = ps.pts[i];
     if (p.kind == kRow && p.live)
@@ -263,12 +268,13 @@ void finish_tile(TileOut &to, PointSet &ps, const std::vector<uint16_t> &corr, R
   }
 }
 
-// Runs work(t, scratch) for every tile on up to 16 threads, one per 16 tiles at
-// most (a thread costs more than a small mesh's tiles).
+// Runs work(t, scratch) for every tile on up to 16 threads, one per kGrain tiles
+// at most (a thread costs more than a small mesh's tiles).
+constexpr size_t kGrain = 6;
 template <typename Scratch, typename F>
 void for_tiles(size_t ntiles, F &&work) {
   const unsigned hw = std::thread::hardware_concurrency();
-  const int nthreads = (int)std::min<size_t>(std::max(1u, std::min(16u, hw ? hw : 1u)), (ntiles + 15) / 16);
+  const int nthreads = (int)std::min<size_t>(std::max(1u, std::min(16u, hw ? hw : 1u)), (ntiles + kGrain - 1) / kGrain);
   std::atomic<size_t> next{0};
   std::exception_ptr err;
   std::mutex mu;
@@ -276,9 +282,9 @@ void for_tiles(size_t ntiles, F &&work) {
     try {
       Scratch sc;
       while (true) {
-        const size_t t0 = next.fetch_add(16);
+        const size_t t0 = next.fetch_add(kGrain);
         if (t0 >= ntiles) break;
-        for (size_t t = t0; t < std::min(ntiles, t0 + 16); t++) work(t, sc);
+        for (size_t t = t0; t < std::min(ntiles, t0 + kGrain); t++) work(t, sc);
       }
     } catch (...) {
       std::lock_guard<std::mutex> g(mu);
@@ -338,6 +344,7 @@ void concatenate(PointHost &o, std::vector<TileOut> &outs, size_t N, int npe) {
     o.max_slots = std::max(o.max_slots, h.npts() + h.ncor + 1);
     o.max_units = std::max(o.max_units, std::max(h.na, h.nb));
     o.max_hang = std::max(o.max_hang, (int)to.hang);
+    o.max_terms = std::max(o.max_terms, 2 * (h.nrow - h.nnode));
     o.max_grp = std::max(o.max_grp, h.ngrp);
     o.entries += to.entries;
     st[0] += h.nrd;
@@ -740,6 +747,173 @@ PointHost build_points_reference(const MeshParams &mp, const Traversal &tr, size
   for_tiles<Scratch>(ntiles, build_tile);
   concatenate(o, outs, N, npe);
   return o;
+}
+
+bool build_points_conforming(const MeshParams &mp, const Traversal &tr, const std::vector<Oct> &nodes, int T,
+                             int max_terms, PointHost &out) {
+  const int dim = mp.dim, npe = tr.nPe;
+  const size_t E = tr.leaves.size(), N = nodes.size();
+  // Node ids by position: open addressing, filled in parallel (positions are
+  // distinct; a node claims the first free slot of its probe sequence).
+  size_t cap = 16;
+  while (cap < 2 * N) cap <<= 1;
+  std::vector<int32_t> table(cap, -1);
+  auto hash = [&](const u32 *x) {
+    u64 h = 0x9E3779B97F4A7C15ull;
+    for (int d = 0; d < dim; d++) h = (h ^ x[d]) * 0xBF58476D1CE4E5B9ull;
+    return (size_t)(h ^ (h >> 31)) & (cap - 1);
+  };
+  constexpr size_t kFill = 2048;  // nodes per unit of work
+  struct None {};
+  for_tiles<None>((N + kFill - 1) / kFill, [&](size_t c, None &) {
+    for (size_t n = c * kFill; n < std::min(N, (c + 1) * kFill); n++)
+      for (size_t i = hash(nodes[n].x);; i = (i + 1) & (cap - 1)) {
+        int32_t free = -1;
+        if (__atomic_compare_exchange_n(&table[i], &free, (int32_t)n, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED)) break;
+      }
+  });
+  auto find_node = [&](const u32 *x) -> int32_t {
+    for (size_t i = hash(x);; i = (i + 1) & (cap - 1)) {
+      const int32_t n = table[i];
+      if (n < 0) return -1;
+      bool same = true;
+      for (int d = 0; same && d < dim; d++) same = nodes[n].x[d] == x[d];
+      if (same) return n;
+    }
+  };
+  const size_t ntiles = (E + T - 1) / T;
+  PointHost o;
+  o.lloc.resize(E * (size_t)npe);
+  o.laux.resize(E);
+  // A position and the level it is resolved from, to its reference.
+  struct Known {
+    struct Key {
+      u32 x[4], lev;
+    };
+    std::vector<Key> key;
+    std::vector<int32_t> ref;
+    std::vector<uint32_t> used;
+    std::vector<uint8_t> full;
+    Known() : key(1 << 14), ref(1 << 14), full(1 << 14, 0) {}
+    void clear() {
+      for (uint32_t u : used) full[u] = 0;
+      used.clear();
+    }
+    // Slot of the key, free or not.
+    uint32_t slot(const Key &k) {
+      u64 h = 0x9E3779B97F4A7C15ull;
+      for (u32 v : {k.x[0], k.x[1], k.x[2], k.x[3], k.lev}) h = (h ^ v) * 0xBF58476D1CE4E5B9ull;
+      uint32_t i = (uint32_t)(h >> 33) & ((1 << 14) - 1);
+      while (full[i] && std::memcmp(&key[i], &k, sizeof k)) i = (i + 1) & ((1 << 14) - 1);
+      return i;
+    }
+    void put(const Key &k, int32_t r) {
+      const uint32_t i = slot(k);
+      if (full[i]) return;
+      if (used.size() * 2 >= full.size()) throw Misfit("tile has too many points");
+      full[i] = 1;
+      key[i] = k;
+      ref[i] = r;
+      used.push_back(i);
+    }
+  };
+  struct Scratch {
+    LocalIds ids;
+    PointSet ps;
+    Renumber rn;
+    Known corner, inside;
+    std::vector<int32_t> ref;
+  };
+  std::vector<TileOut> outs(ntiles);
+  auto build_tile = [&](size_t t, Scratch &sc) {
+    TileOut &to = outs[t];
+    const size_t l0 = t * T, l1 = std::min(E, l0 + T);
+    to.h.leaf0 = (int32_t)l0;
+    to.h.nleaf = (int32_t)(l1 - l0);
+    sc.ids.clear();
+    sc.ps.clear();
+    sc.corner.clear();
+    sc.inside.clear();
+    sc.ref.assign((l1 - l0) * npe, 0);
+    auto node = [&](int32_t n) -> int32_t {
+      bool fresh;
+      const int32_t l = sc.ids.get(n, &fresh);
+      if (fresh) {
+        to.nodes.push_back(n);
+        to.is_target.push_back(1);
+      }
+      return l;
+    };
+    // interpolant: the value at x of the cell (anchor a, level lev); cornered: at
+    // a corner of that cell, a node or the interpolant of its parent.
+    auto cornered = [&](auto &&self, auto &&inside, const u32 *x, const u32 *a, u32 lev) -> int32_t {
+      typename Known::Key k{{x[0], x[1], x[2], x[3]}, lev};
+      const uint32_t i = sc.corner.slot(k);
+      if (sc.corner.full[i]) return sc.corner.ref[i];
+      int32_t r;
+      if (const int32_t n = find_node(x); n >= 0) {
+        r = node(n);
+      } else {
+        if (lev == 0) throw std::runtime_error("conforming constraint: a root node is missing");
+        const u32 plen = 2u << (mp.maxd - lev);
+        u32 pa[4] = {0, 0, 0, 0};
+        for (int d = 0; d < dim; d++) pa[d] = a[d] & ~(plen - 1);
+        r = inside(self, inside, x, pa, lev - 1);
+      }
+      sc.corner.put(k, r);
+      return r;
+    };
+    auto inside = [&](auto &&cornered, auto &&self, const u32 *x, const u32 *a, u32 lev) -> int32_t {
+      const u32 len = 1u << (mp.maxd - lev);
+      int d = dim - 1;  // the last axis on which x is no end of the cell
+      while (d >= 0 && (x[d] == a[d] || x[d] == a[d] + len)) d--;
+      if (d < 0) return cornered(cornered, self, x, a, lev);
+      // Known by position and level: cells of one level that share the position
+      // share the face behind it.
+      typename Known::Key k{{x[0], x[1], x[2], x[3]}, lev};
+      const uint32_t i = sc.inside.slot(k);
+      if (sc.inside.full[i]) return sc.inside.ref[i];
+      u32 xa[4] = {x[0], x[1], x[2], x[3]}, xb[4] = {x[0], x[1], x[2], x[3]};
+      xa[d] = a[d];
+      xb[d] = a[d] + len;
+      const int32_t ra = self(cornered, self, xa, a, lev), rb = self(cornered, self, xb, a, lev);
+      const uint16_t none = 0;
+      const int32_t r = -1 - sc.ps.add(kRow, 1, ra, rb, &none, 0, &none, 0);
+      sc.inside.put(k, r);
+      return r;
+    };
+    for (size_t e = l0; e < l1; e++) {
+      const Oct &c = tr.leaves[e];
+      const u32 len = 1u << (mp.maxd - c.lev);
+      for (int r = 0; r < npe; r++) {
+        const int32_t n = tr.slot[e * npe + r];
+        int32_t &ref = sc.ref[(e - l0) * npe + r];
+        if (n >= 0) {
+          ref = node(n);
+          continue;
+        }
+        u32 x[4] = {0, 0, 0, 0}, pa[4] = {0, 0, 0, 0};
+        for (int d = 0; d < dim; d++) {
+          x[d] = c.x[d] + ((r >> d) & 1) * len;
+          pa[d] = c.x[d] & ~(2 * len - 1);
+        }
+        ref = inside(cornered, inside, x, pa, c.lev - 1);
+        if (ref < 0) sc.ps.pts[-1 - ref].live = true;
+      }
+      o.laux[e] = (c.lev & 31u) | ((uint32_t)tr.child[e] << 5);
+    }
+    finish_tile(to, sc.ps, {}, sc.rn);
+    if (2 * (to.h.nrow - to.h.nnode) > max_terms) throw Misfit("tile has too many row ends");
+    for (size_t i = 0; i < (l1 - l0) * npe; i++) o.lloc[l0 * npe + i] = sc.rn(sc.ref[i]);
+  };
+  try {
+    for_tiles<Scratch>(ntiles, build_tile);
+  } catch (const Misfit &) {
+    return false;
+  }
+  concatenate(o, outs, N, npe);
+  out = std::move(o);
+  return true;
 }
 
 }  // namespace dkt

@@ -78,6 +78,7 @@ struct PointHost {
   std::vector<uint16_t> lloc;
   std::vector<uint32_t> laux;
   int max_nodes = 0, max_slots = 0, max_units = 0, max_hang = 0;
+  int max_terms = 0;          // ends of rows (two each)
   int max_grp = 0;            // sibling groups of a replay (0: no tile has readers)
   size_t npartial = 0;
   size_t entries = 0;         // transposed terms (without the padding)
@@ -88,5 +89,13 @@ struct PointHost {
 // Reference semantics over the flattened traversal, tiles of at most T leaves;
 // n_groups: replay blocks per tile.
 PointHost build_points_reference(const MeshParams &mp, const Traversal &tr, size_t N, int T, int n_groups);
+
+// Conforming operator (sum_e C_e^T K_e C_e, build_conforming): a rank that is no
+// node takes its parent cell's interpolant, whose corners do the same one level
+// up, so every hanging point is a row.  Tiles of T elements.  Returns false where
+// a tile does not fit the layout (more row levels than kPtLevels, or more than
+// max_terms ends of rows).
+bool build_points_conforming(const MeshParams &mp, const Traversal &tr, const std::vector<Oct> &nodes, int T,
+                             int max_terms, PointHost &out);
 
 }  // namespace dkt
