@@ -49,58 +49,89 @@ enum { S_RR0 = 0, S_RR1 = 1, S_NORMB = 2, S_RESID = 3, S_SCALE = 4, S_BETA = 5, 
 // Stop reasons in flag[0] (0: running), as reported in the solve statistics.
 constexpr int kStopConverged = 1, kStopMaxIter = 2, kStopBreakdown = 3, kStopStalled = 4;
 
-template <typename T>
-__device__ __forceinline__ T block_sum(T v, T *sh) {
-  const int t = threadIdx.x;
-  __syncthreads();
-  sh[t] = v;
-  __syncthreads();
-#pragma unroll
-  for (int s = kCgThreads / 2; s > 0; s >>= 1) {
-    if (t < s) sh[t] += sh[t + s];
-    __syncthreads();
-  }
-  return sh[0];
+// Sum and max over a wavefront, in every lane, in a fixed order: lane moves
+// inside rows of 16 (no LDS), then across the rows.
+__device__ __forceinline__ double wave_sum(double v) {
+  v += xor_lane<0>(v);
+  v += xor_lane<1>(v);
+  v += xor_lane<2>(v);
+  v += xor_lane<3>(v);
+  v += __shfl_xor(v, 16, 64);
+  v += __shfl_xor(v, 32, 64);
+  return v;
+}
+__device__ __forceinline__ double wave_max(double v) {
+  v = fmax(v, xor_lane<0>(v));
+  v = fmax(v, xor_lane<1>(v));
+  v = fmax(v, xor_lane<2>(v));
+  v = fmax(v, xor_lane<3>(v));
+  v = fmax(v, __shfl_xor(v, 16, 64));
+  v = fmax(v, __shfl_xor(v, 32, 64));
+  return v;
 }
 
-template <typename T>
-__device__ __forceinline__ T block_max(T v, T *sh) {
-  const int t = threadIdx.x;
+// Sum s and max m over the block, in every work-item.
+constexpr int kCgWaves = kCgThreads / 64;
+static_assert(kCgWaves == 4, "the reductions add four wavefronts");
+__device__ __forceinline__ void block_sum_max(double &s, double &m, double *sh) {
+  s = wave_sum(s);
+  m = wave_max(m);
+  const int w = threadIdx.x >> 6;
   __syncthreads();
-  sh[t] = v;
-  __syncthreads();
-#pragma unroll
-  for (int s = kCgThreads / 2; s > 0; s >>= 1) {
-    if (t < s) sh[t] = fmax(sh[t], sh[t + s]);
-    __syncthreads();
+  if (!(threadIdx.x & 63)) {
+    sh[w] = s;
+    sh[kCgWaves + w] = m;
   }
-  return sh[0];
+  __syncthreads();
+  s = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+  m = fmax(fmax(sh[4], sh[5]), fmax(sh[6], sh[7]));
+}
+__device__ __forceinline__ double block_sum(double v, double *sh) {
+  v = wave_sum(v);
+  __syncthreads();
+  if (!(threadIdx.x & 63)) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+__device__ __forceinline__ double block_max(double v, double *sh) {
+  v = wave_max(v);
+  __syncthreads();
+  if (!(threadIdx.x & 63)) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return fmax(fmax(sh[0], sh[1]), fmax(sh[2], sh[3]));
 }
 
 // Sum (or max) of the kCgBlocks partials, identical in every block.
-__device__ __forceinline__ double parts_sum(const double *part, double *sh) {
-  return block_sum(part[threadIdx.x] + part[threadIdx.x + kCgThreads], sh);
+__device__ __forceinline__ double parts_of(const double *part) {
+  return part[threadIdx.x] + part[threadIdx.x + kCgThreads];
 }
-__device__ __forceinline__ double parts_max(const double *part, double *sh) {
-  return block_max(fmax(part[threadIdx.x], part[threadIdx.x + kCgThreads]), sh);
+__device__ __forceinline__ double parts_top(const double *part) {
+  return fmax(part[threadIdx.x], part[threadIdx.x + kCgThreads]);
 }
+__device__ __forceinline__ double parts_sum(const double *part, double *sh) { return block_sum(parts_of(part), sh); }
+__device__ __forceinline__ double parts_max(const double *part, double *sh) { return block_max(parts_top(part), sh); }
 
-// Blocks of a solve over n entries: at least 4 entries per work-item, at most
-// kCgBlocks.  Blocks past it write no partials; the partial arrays keep zeros
+// Blocks of a solve over n entries: one entry per work-item up to kCgBlocks (a
+// small solve's kernels are as long as the chain of one work-item: 10,000 unknowns
+// on 40 blocks instead of 10, four entries each, took 1 to 2 us less a kernel).  Blocks past it write no partials; the partial arrays keep zeros
 // there (zeroed with the workspace), which the fixed-order sums and max norms
 // over all kCgBlocks slots ignore.
 __host__ __device__ inline int cg_blocks(int n) {
-  const int b = (n + 4 * kCgThreads - 1) / (4 * kCgThreads);
+  const int b = (n + kCgThreads - 1) / kCgThreads;
   return b < 1 ? 1 : (b > kCgBlocks ? kCgBlocks : b);
 }
 #define CG_LOOP(i, n) \
   for (int i = blockIdx.x * kCgThreads + threadIdx.x; i < (n); i += cg_blocks(n) * kCgThreads)
 
-// The iteration kernels' loops take kCgUnroll of a work-item's entries at a
-// time with every load issued before any use (one memory round trip per batch
-// where the plain loop waits once per entry), then handle them in index order:
-// each work-item's sums keep the order, and the bits, of the plain loop.
+// The iteration kernels handle a work-item's entries kCgUnroll at a time, every
+// load of a batch issued before any use.  What a kernel needs before its first
+// batch (the stop flag, the partials of the last reduction) is loaded with it, and
+// a stopped solve's kernels run through without writing, instead of each load
+// waiting for the test before it: below a few hundred thousand unknowns a kernel
+// is a chain of memory round trips and reductions and nothing else.
 constexpr int kCgUnroll = 4;
+#define CG_BATCH(u, k, i) \
+  _Pragma("unroll") for (int u = 0, k = (i); u < kCgUnroll; u++, k += stride)
 
 // The bodies of the iteration kernels run one solve's block blockIdx.x of
 // kCgBlocks; the single-solve kernels and the batched ones (one solve per
@@ -111,7 +142,7 @@ constexpr int kCgUnroll = 4;
 template <typename T>
 __device__ __forceinline__ void init_body(int n, const T *__restrict__ b, const T *__restrict__ ax,
                                           T *__restrict__ r, T *__restrict__ p, double *__restrict__ part) {
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   double rr = 0, mr = 0, mb = 0;
   CG_LOOP(i, n) {
     const T ri = ax ? b[i] - ax[i] : b[i];
@@ -121,8 +152,7 @@ __device__ __forceinline__ void init_body(int n, const T *__restrict__ b, const 
     mr = fmax(mr, (double)fabs(ri));
     mb = fmax(mb, (double)fabs(b[i]));
   }
-  rr = block_sum(rr, sh);
-  mr = block_max(mr, sh);
+  block_sum_max(rr, mr, sh);
   mb = block_max(mb, sh);
   if (threadIdx.x == 0) {
     part[blockIdx.x] = rr;
@@ -138,7 +168,7 @@ __global__ void __launch_bounds__(kCgThreads) k_init(int n, const T *__restrict_
 
 __device__ __forceinline__ void init_fin_body(const double *__restrict__ part, double *__restrict__ scal, double tol,
                                               int *__restrict__ flag) {
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   const double rr = parts_sum(part, sh);
   const double mr = parts_max(part + kCgBlocks, sh);
   double mb = parts_max(part + 2 * kCgBlocks, sh);
@@ -159,24 +189,21 @@ __global__ void __launch_bounds__(kCgThreads) k_init_fin(const double *__restric
 template <typename T>
 __device__ __forceinline__ void dot_body(int n, const T *__restrict__ a, const T *__restrict__ b,
                                          double *__restrict__ part, const int *__restrict__ flag) {
-  if (flag[0]) return;
-  __shared__ double sh[kCgThreads];
-  double acc = 0;
+  __shared__ double sh[2 * kCgWaves];
+  const bool run = !flag[0];
   const int stride = cg_blocks(n) * kCgThreads;
-  int i = blockIdx.x * kCgThreads + threadIdx.x;
-  for (; i < n - (kCgUnroll - 1) * stride; i += kCgUnroll * stride) {
+  double acc = 0;
+  for (int i = blockIdx.x * kCgThreads + threadIdx.x; i < n; i += kCgUnroll * stride) {
     T av[kCgUnroll], bv[kCgUnroll];
-#pragma unroll
-    for (int u = 0; u < kCgUnroll; u++) {
-      av[u] = a[i + u * stride];
-      bv[u] = b[i + u * stride];
+    CG_BATCH(u, k, i) {
+      av[u] = k < n ? a[k] : T(0);
+      bv[u] = k < n ? b[k] : T(0);
     }
-#pragma unroll
-    for (int u = 0; u < kCgUnroll; u++) acc += (double)av[u] * (double)bv[u];
+    CG_BATCH(u, k, i) acc += (double)av[u] * (double)bv[u];
+    if (!run) break;
   }
-  for (; i < n; i += stride) acc += (double)a[i] * (double)b[i];
   acc = block_sum(acc, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = acc;
+  if (run && threadIdx.x == 0) part[blockIdx.x] = acc;
 }
 template <typename T>
 __global__ void __launch_bounds__(kCgThreads) k_dot(int n, const T *__restrict__ a, const T *__restrict__ b,
@@ -190,51 +217,50 @@ __device__ __forceinline__ void update_xr_body(int n, T *__restrict__ x, T *__re
                                                const T *__restrict__ ap, const double *__restrict__ part_pap,
                                                const double *__restrict__ scal, int par, double *__restrict__ part,
                                                int *__restrict__ flag) {
-  if (flag[0]) return;
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
+  bool run = !flag[0];
+  const double rr0 = scal[S_RR0 + par];
+  double pap = parts_of(part_pap);
+  const int stride = cg_blocks(n) * kCgThreads;
+  int i = blockIdx.x * kCgThreads + threadIdx.x;
+  T xv[kCgUnroll], pv[kCgUnroll], rv[kCgUnroll], av[kCgUnroll];
+  auto load = [&]() {
+    CG_BATCH(u, k, i) {
+      const int j = k < n ? k : 0;
+      xv[u] = x[j];
+      pv[u] = p[j];
+      rv[u] = r[j];
+      av[u] = ap[j];
+    }
+  };
+  load();
   // Breakdown guard: p.Ap <= 0 (the operator is not positive definite on p)
   // or a non-finite step stops the solve before x or r change.  Every block
   // reduces the same partials in the same order, so all of them agree.
-  const double pap = parts_sum(part_pap, sh);
-  const double a64 = scal[S_RR0 + par] / pap;
-  if (!(pap > 0.0) || !isfinite(a64)) {
+  pap = block_sum(pap, sh);
+  const double a64 = rr0 / pap;
+  if (run && (!(pap > 0.0) || !isfinite(a64))) {
     if (blockIdx.x == 0 && threadIdx.x == 0) flag[0] = kStopBreakdown;
-    return;
+    run = false;
   }
   const T alpha = (T)a64;
   double rr = 0, mr = 0;
-  const int stride = cg_blocks(n) * kCgThreads;
-  int i = blockIdx.x * kCgThreads + threadIdx.x;
-  for (; i < n - (kCgUnroll - 1) * stride; i += kCgUnroll * stride) {
-    T xv[kCgUnroll], pv[kCgUnroll], rv[kCgUnroll], av[kCgUnroll];
-#pragma unroll
-    for (int u = 0; u < kCgUnroll; u++) {
-      const int k = i + u * stride;
-      xv[u] = x[k];
-      pv[u] = p[k];
-      rv[u] = r[k];
-      av[u] = ap[k];
+  const int m = run ? n : 0;
+  while (i < m) {
+    CG_BATCH(u, k, i) {
+      if (k < m) {
+        x[k] = xv[u] + alpha * pv[u];
+        const T ri = rv[u] - alpha * av[u];
+        r[k] = ri;
+        rr += (double)ri * (double)ri;
+        mr = fmax(mr, (double)fabs(ri));
+      }
     }
-#pragma unroll
-    for (int u = 0; u < kCgUnroll; u++) {
-      const int k = i + u * stride;
-      x[k] = xv[u] + alpha * pv[u];
-      const T ri = rv[u] - alpha * av[u];
-      r[k] = ri;
-      rr += (double)ri * (double)ri;
-      mr = fmax(mr, (double)fabs(ri));
-    }
+    i += kCgUnroll * stride;
+    if (i < m) load();
   }
-  for (; i < n; i += stride) {
-    x[i] += alpha * p[i];
-    const T ri = r[i] - alpha * ap[i];
-    r[i] = ri;
-    rr += (double)ri * (double)ri;
-    mr = fmax(mr, (double)fabs(ri));
-  }
-  rr = block_sum(rr, sh);
-  mr = block_max(mr, sh);
-  if (threadIdx.x == 0) {
+  block_sum_max(rr, mr, sh);
+  if (run && threadIdx.x == 0) {
     part[blockIdx.x] = rr;
     part[kCgBlocks + blockIdx.x] = mr;
   }
@@ -250,38 +276,46 @@ __global__ void __launch_bounds__(kCgThreads) k_update_xr(int n, T *__restrict__
 
 // Convergence test, then beta = r1.r1 / r0.r0 and p = r + beta p.  Block 0
 // publishes the new r.r (into the other parity slot), the residual, the
-// iteration count and the converged flag.
+// iteration count and the converged flag.  Returns whether the solve was
+// running.
 template <typename T>
-__device__ __forceinline__ void update_p_body(int n, T *__restrict__ p, const T *__restrict__ r,
+__device__ __forceinline__ bool update_p_body(int n, T *__restrict__ p, const T *__restrict__ r,
                                               const double *__restrict__ part, double *__restrict__ scal, int par,
                                               double tol, int *__restrict__ flag) {
-  if (flag[0]) return;
-  __shared__ double sh[kCgThreads];
-  const double rr1 = parts_sum(part, sh);
-  const double resid = parts_max(part + kCgBlocks, sh) / scal[S_NORMB];
-  const bool done = resid <= tol;
-  if (!done) {
-    const T beta = (T)(rr1 / scal[S_RR0 + par]);
-    const int stride = cg_blocks(n) * kCgThreads;
-    int i = blockIdx.x * kCgThreads + threadIdx.x;
-    for (; i < n - (kCgUnroll - 1) * stride; i += kCgUnroll * stride) {
-      T rv[kCgUnroll], pv[kCgUnroll];
-#pragma unroll
-      for (int u = 0; u < kCgUnroll; u++) {
-        rv[u] = r[i + u * stride];
-        pv[u] = p[i + u * stride];
-      }
-#pragma unroll
-      for (int u = 0; u < kCgUnroll; u++) p[i + u * stride] = rv[u] + beta * pv[u];
+  __shared__ double sh[2 * kCgWaves];
+  const bool run = !flag[0];
+  const double rr0 = scal[S_RR0 + par], normb = scal[S_NORMB];
+  double rr1 = parts_of(part), top = parts_top(part + kCgBlocks);
+  const int stride = cg_blocks(n) * kCgThreads;
+  int i = blockIdx.x * kCgThreads + threadIdx.x;
+  T rv[kCgUnroll], pv[kCgUnroll];
+  auto load = [&]() {
+    CG_BATCH(u, k, i) {
+      const int j = k < n ? k : 0;
+      rv[u] = r[j];
+      pv[u] = p[j];
     }
-    for (; i < n; i += stride) p[i] = r[i] + beta * p[i];
+  };
+  load();
+  block_sum_max(rr1, top, sh);
+  const double resid = top / normb;
+  const bool done = resid <= tol;
+  const T beta = (T)(rr1 / rr0);
+  const int m = run && !done ? n : 0;
+  while (i < m) {
+    CG_BATCH(u, k, i) {
+      if (k < m) p[k] = rv[u] + beta * pv[u];
+    }
+    i += kCgUnroll * stride;
+    if (i < m) load();
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  if (run && blockIdx.x == 0 && threadIdx.x == 0) {
     scal[S_RR0 + (par ^ 1)] = rr1;
     scal[S_RESID] = resid;
     flag[1] += 1;
     if (done) flag[0] = 1;
   }
+  return run;
 }
 template <typename T>
 __global__ void __launch_bounds__(kCgThreads) k_update_p(int n, T *__restrict__ p, const T *__restrict__ r,
@@ -294,7 +328,7 @@ __global__ void __launch_bounds__(kCgThreads) k_update_p(int n, T *__restrict__ 
 __global__ void __launch_bounds__(kCgThreads) k_resid64(int n, const double *__restrict__ b,
                                                         const double *__restrict__ ax, double *__restrict__ r,
                                                         double *__restrict__ part) {
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   double mr = 0, mb = 0;
   CG_LOOP(i, n) {
     const double ri = b[i] - ax[i];
@@ -312,7 +346,7 @@ __global__ void __launch_bounds__(kCgThreads) k_resid64(int n, const double *__r
 
 // scal[S_RESID] = max|r| / max|b| (max|b| = 1 if b = 0); scal[S_SCALE] = max|r|.
 __global__ void __launch_bounds__(kCgThreads) k_resid64_fin(const double *__restrict__ part, double *__restrict__ scal) {
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   const double mr = parts_max(part, sh);
   double mb = parts_max(part + kCgBlocks, sh);
   if (threadIdx.x == 0) {
@@ -354,7 +388,7 @@ __global__ void __launch_bounds__(kCgThreads) k_add32u(int n, double *__restrict
 __global__ void __launch_bounds__(kCgThreads) k_rel32(int n, const double *__restrict__ r64, float *__restrict__ r32,
                                                       float *__restrict__ p32, float *__restrict__ x32, int restart,
                                                       double *__restrict__ part) {
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   double rr = 0;
   CG_LOOP(i, n) {
     const float ri = (float)r64[i];
@@ -374,7 +408,7 @@ __global__ void __launch_bounds__(kCgThreads) k_rel32(int n, const double *__res
 __global__ void __launch_bounds__(kCgThreads) k_rel32_fin(const double *__restrict__ part, double *__restrict__ scal32,
                                                           const double *__restrict__ scal64, int par, int restart,
                                                           int *__restrict__ flag) {
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   const double rr = parts_sum(part, sh);
   if (threadIdx.x == 0) {
     scal32[S_BETA] = restart ? 0.0 : rr / scal32[S_RR0 + par];
@@ -618,9 +652,9 @@ __global__ void __launch_bounds__(kCgThreads) kb_update_xr(const CgDesc<T> *__re
 template <typename T>
 __global__ void __launch_bounds__(kCgThreads) kb_update_p(const CgDesc<T> *__restrict__ d, int par) {
   const CgDesc<T> e = d[blockIdx.y];
-  if (blockIdx.x >= cg_blocks(e.n) || e.flag[0]) return;
-  update_p_body<T>(e.n, e.p, e.r, e.part, e.scal, par, e.tolp ? *e.tolp : e.tol, e.flag);
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  if (blockIdx.x >= cg_blocks(e.n)) return;
+  const bool run = update_p_body<T>(e.n, e.p, e.r, e.part, e.scal, par, e.tolp ? *e.tolp : e.tol, e.flag);
+  if (run && blockIdx.x == 0 && threadIdx.x == 0) {
     if (!e.flag[0] && e.flag[1] >= e.max_iter) e.flag[0] = kStopMaxIter;
     if (e.flag[0]) e.scal[S_PAR] = par;
   }
@@ -669,7 +703,7 @@ __global__ void __launch_bounds__(kCgThreads) kr_resid(const RelDesc *__restrict
         e.part64[j] = 0.0;
         e.part32[j] = 0.0;
       }
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   double mr = 0, mb = 0;
   CG_LOOP(i, e.n) {
     const double ri = u == 2 ? e.b[i] : e.b[i] - e.ap64[i];
@@ -689,7 +723,7 @@ __global__ void __launch_bounds__(kCgThreads) kr_decide(const RelDesc *__restric
   const RelDesc e = d[blockIdx.y];
   const int u = *e.upd;
   if (!u) return;
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   const double mr = parts_max(e.part64, sh);
   double mb = parts_max(e.part64 + kCgBlocks, sh);
   if (threadIdx.x != 0) return;
@@ -739,7 +773,7 @@ __global__ void __launch_bounds__(kCgThreads) kr_rel32(const RelDesc *__restrict
   const RelDesc e = d[blockIdx.y];
   if (!*e.upd || e.flag[0] || blockIdx.x >= cg_blocks(e.n)) return;
   const bool restart = e.st[3] != 0.0;
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   double rr = 0;
   CG_LOOP(i, e.n) {
     const float ri = (float)e.r64[i];
@@ -755,7 +789,7 @@ __global__ void __launch_bounds__(kCgThreads) kr_rel32(const RelDesc *__restrict
 __global__ void __launch_bounds__(kCgThreads) kr_rel32_fin(const RelDesc *__restrict__ d) {
   const RelDesc e = d[blockIdx.y];
   if (!*e.upd || e.flag[0]) return;
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   const double rr = parts_sum(e.part32, sh);
   if (threadIdx.x == 0) {
     const int par = *e.upd == 2 ? 0 : (int)e.scal32[S_PAR];
@@ -804,7 +838,7 @@ struct BiVecs {
 // r = b - ax, r^ = r, p = v = 0; partials of r.r, max|r|, max|b|.
 __global__ void __launch_bounds__(kCgThreads) kbi_init(int n, const double *__restrict__ b,
                                                        const double *__restrict__ ax, BiVecs w) {
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   double rr = 0, mr = 0, mb = 0;
   CG_LOOP(i, n) {
     const double ri = b[i] - ax[i];
@@ -816,8 +850,7 @@ __global__ void __launch_bounds__(kCgThreads) kbi_init(int n, const double *__re
     mr = fmax(mr, fabs(ri));
     mb = fmax(mb, fabs(b[i]));
   }
-  rr = block_sum(rr, sh);
-  mr = block_max(mr, sh);
+  block_sum_max(rr, mr, sh);
   mb = block_max(mb, sh);
   if (threadIdx.x == 0) {
     w.part[blockIdx.x] = rr;
@@ -826,7 +859,7 @@ __global__ void __launch_bounds__(kCgThreads) kbi_init(int n, const double *__re
   }
 }
 __global__ void __launch_bounds__(kCgThreads) kbi_init_fin(BiVecs w, double tol, int *__restrict__ flag) {
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   const double rr = parts_sum(w.part, sh);
   const double mr = parts_max(w.part + kCgBlocks, sh);
   double mb = parts_max(w.part + 2 * kCgBlocks, sh);
@@ -854,7 +887,7 @@ __global__ void __launch_bounds__(kCgThreads) kbi_dot(int n, const double *__res
                                                       const double *__restrict__ c, const double *__restrict__ d,
                                                       double *__restrict__ part, const int *__restrict__ flag) {
   if (flag[0]) return;
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   double ab = 0, cd = 0;
   CG_LOOP(i, n) {
     ab += a[i] * b[i];
@@ -870,7 +903,7 @@ __global__ void __launch_bounds__(kCgThreads) kbi_dot(int n, const double *__res
 // alpha = rho / (r^.v); s = r - alpha v.  r^.v = 0 or a non-finite alpha: breakdown.
 __global__ void __launch_bounds__(kCgThreads) kbi_s(int n, BiVecs w, int *__restrict__ flag) {
   if (flag[0]) return;
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   const double rv = parts_sum(w.part + 3 * kCgBlocks, sh);
   const double alpha = w.scal[B_RHO] / rv;
   if (!(rv != 0.0) || !isfinite(alpha)) {
@@ -885,7 +918,7 @@ __global__ void __launch_bounds__(kCgThreads) kbi_s(int n, BiVecs w, int *__rest
 __global__ void __launch_bounds__(kCgThreads) kbi_xr(int n, double *__restrict__ x, BiVecs w,
                                                      const int *__restrict__ flag) {
   if (flag[0]) return;
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   const double ts = parts_sum(w.part + 4 * kCgBlocks, sh);
   const double tt = parts_sum(w.part + 5 * kCgBlocks, sh);
   const double om = tt > 0.0 ? ts / tt : 0.0;
@@ -898,8 +931,7 @@ __global__ void __launch_bounds__(kCgThreads) kbi_xr(int n, double *__restrict__
     rr += w.rh[i] * ri;
     mr = fmax(mr, fabs(ri));
   }
-  rr = block_sum(rr, sh);
-  mr = block_max(mr, sh);
+  block_sum_max(rr, mr, sh);
   if (threadIdx.x == 0) {
     w.part[blockIdx.x] = rr;
     w.part[kCgBlocks + blockIdx.x] = mr;
@@ -910,7 +942,7 @@ __global__ void __launch_bounds__(kCgThreads) kbi_xr(int n, double *__restrict__
 // 0 with the residual above tol: breakdown (the next beta is undefined).
 __global__ void __launch_bounds__(kCgThreads) kbi_fin(BiVecs w, double tol, int max_iter, int *__restrict__ flag) {
   if (flag[0]) return;
-  __shared__ double sh[kCgThreads];
+  __shared__ double sh[2 * kCgWaves];
   const double rho = parts_sum(w.part, sh);
   const double mr = parts_max(w.part + kCgBlocks, sh);
   if (threadIdx.x == 0) {

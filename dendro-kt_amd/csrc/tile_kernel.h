@@ -88,29 +88,6 @@ __host__ __device__ inline size_t tile_region_bytes(const TileDims &D) {
   return m > 16 ? m : 16;
 }
 
-// Cross-lane moves inside a row of 16 lanes (DPP, a VALU operand modifier;
-// no LDS round trip).  Controls: quad_perm [1,0,3,2] = 0xB1, [2,3,0,1] = 0x4E,
-// [3,2,1,0] = 0x1B, row_half_mirror = 0x141, row_ror:8 = 0x128.
-template <int CTRL>
-__device__ __forceinline__ float dpp_mov(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
-}
-template <int CTRL>
-__device__ __forceinline__ double dpp_mov(double v) {
-  const long long u = __builtin_bit_cast(long long, v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(u & 0xFFFFFFFFll), CTRL, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, 0xF, 0xF, true);
-  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
-}
-// Value of lane (lane ^ (1 << D)) within the same row of 16.
-template <int D, typename T>
-__device__ __forceinline__ T xor_lane(T a) {
-  if constexpr (D == 0) return dpp_mov<0xB1>(a);
-  else if constexpr (D == 1) return dpp_mov<0x4E>(a);
-  else if constexpr (D == 2) return dpp_mov<0x1B>(dpp_mov<0x141>(a));  // (lane ^ 7) ^ 3
-  else return dpp_mov<0x128>(a);
-}
-
 // One step of the sibling-group sum: w[s] += (value of lane wl + D in the same
 // row of 16) when that lane is still in the run.  Products with the 0/1 factor
 // are exact, so the fma adds an exact zero or rounds once like the plain sum.
