@@ -135,13 +135,11 @@ struct Group : GroupBase, FixSource<T> {
     auto dims_of = [](const dkt_plan *pl) {
       return TileDims{pl->max_nodes, pl->max_grp, pl->max_he, pl->max_rd, pl->max_cr, pl->tile_leaves, pl->max_hang};
     };
-    // Columns per launch: the most every plan's tiles fit in LDS.
-    // Column-major vectors ([nrhs][N]): one contiguous column per launch.
-    int chunk = colmajor ? 1 : (max_cols > 0 ? std::min(nrhs, max_cols) : nrhs);
-    for (dkt_plan *pl : pls) {
-      if (tile_lds_bytes<T, NPE>(dims_of(pl), 1) > kLdsLimit) throw std::invalid_argument("tile does not fit in LDS");
-      while (chunk > 1 && tile_lds_bytes<T, NPE>(dims_of(pl), chunk) > kLdsLimit) chunk--;
-    }
+    // Columns of a record, separate items of the launch; column-major vectors
+    // ([nrhs][N]) take one record per column.
+    const int chunk = colmajor ? 1 : (max_cols > 0 ? std::min(nrhs, max_cols) : nrhs);
+    for (dkt_plan *pl : pls)
+      if (tile_lds_bytes<T, NPE>(dims_of(pl)) > kLdsLimit) throw std::invalid_argument("tile does not fit in LDS");
     const int nchunks = (nrhs + chunk - 1) / chunk;
     std::vector<int> ts{0};
     std::vector<size_t> poff;
@@ -151,7 +149,7 @@ struct Group : GroupBase, FixSource<T> {
         threads = std::max(threads, pl->tile_leaves);
         poff.push_back(ptot);
         ptot += pl->npartial * (size_t)chunk;
-        ts.push_back(ts.back() + (int)pl->ntiles);
+        ts.push_back(ts.back() + (int)pl->ntiles * std::min(chunk, nrhs - c * chunk));
       }
     partial = mem.alloc<T>(std::max<size_t>(1, ptot));
     one = chunk == 1;
@@ -161,7 +159,7 @@ struct Group : GroupBase, FixSource<T> {
       for (size_t k = 0; k < pls.size(); k++) {
         dkt_plan *pl = pls[k];
         BatchPlan<T> &r = hp[c * pls.size() + k];
-        lds = std::max(lds, tile_lds_bytes<T, NPE>(dims_of(pl), nq));
+        lds = std::max(lds, tile_lds_bytes<T, NPE>(dims_of(pl)));
         TileArgs &A = r.A;
         A.tiles = pl->tiles.p;
         A.tile_nodes = pl->tile_nodes.p;
@@ -202,12 +200,9 @@ struct Group : GroupBase, FixSource<T> {
   }
 
   void launch(hipStream_t st) override {
-    if (ntiles && one)
-      hipLaunchKernelGGL((tile_kernel_batch<T, DIM, P, true>), dim3(ntiles), dim3(threads), lds, st, table,
-                         tile_start, nrec);
-    else if (ntiles)
-      hipLaunchKernelGGL((tile_kernel_batch<T, DIM, P, false>), dim3(ntiles), dim3(threads), lds, st, table,
-                         tile_start, nrec);
+    if (ntiles)
+      hipLaunchKernelGGL((one ? tile_kernel_batch<T, DIM, P, true> : tile_kernel_batch<T, DIM, P, false>),
+                         dim3(ntiles), dim3(threads), lds, st, table, tile_start, nrec);
     HIP_OK(hipGetLastError());
   }
 };
@@ -309,8 +304,8 @@ __global__ void __launch_bounds__(kTileThreads) conf_tile_kernel_batch(const Con
 }
 
 // Conforming plans of one (dim, p) (CAP: with per-level captured matrices):
-// one tile launch and one fix-up launch, with one record per (column chunk
-// that fits the tiles' LDS, plan).  Each result is bitwise the plan's own
+// one tile launch and one fix-up launch, with one record per (column chunk,
+// plan).  Each result is bitwise the plan's own
 // matvec (same tile work, same fix-up order).
 template <typename T, int DIM, int P, bool CAP>
 struct ConfGroup : GroupBase, FixSource<T> {
@@ -327,12 +322,10 @@ struct ConfGroup : GroupBase, FixSource<T> {
     mem.arena = arena;
     constexpr int NPE = Pow<P + 1, DIM>::v;
     const bool f64 = sizeof(T) == 8;
-    auto lds_of = [](const dkt_plan *pl, int nq) { return conf_lds_bytes<T, NPE>(pl->max_nodes, nq, pl->nw); };
-    int chunk = colmajor ? 1 : (max_cols > 0 ? std::min(nrhs, max_cols) : nrhs);
-    for (dkt_plan *pl : pls) {
-      if (lds_of(pl, 1) > kLdsLimit) throw std::invalid_argument("tile does not fit in LDS");
-      while (chunk > 1 && lds_of(pl, chunk) > kLdsLimit) chunk--;
-    }
+    auto lds_of = [](const dkt_plan *pl) { return conf_lds_bytes<T, NPE>(pl->max_nodes, pl->nw); };
+    const int chunk = colmajor ? 1 : (max_cols > 0 ? std::min(nrhs, max_cols) : nrhs);
+    for (dkt_plan *pl : pls)
+      if (lds_of(pl) > kLdsLimit) throw std::invalid_argument("tile does not fit in LDS");
     const int nchunks = (nrhs + chunk - 1) / chunk;
     std::vector<int> ts{0};
     std::vector<size_t> poff;
@@ -342,7 +335,7 @@ struct ConfGroup : GroupBase, FixSource<T> {
         threads = std::max(threads, pl->tile_leaves);
         poff.push_back(ptot);
         ptot += pl->npartial * (size_t)chunk;
-        ts.push_back(ts.back() + (int)pl->ntiles);
+        ts.push_back(ts.back() + (int)pl->ntiles * std::min(chunk, nrhs - c * chunk));
       }
     partial = mem.alloc<T>(std::max<size_t>(1, ptot));
     std::vector<ConfBatchPlan<T>> hp(pls.size() * nchunks);
@@ -353,7 +346,7 @@ struct ConfGroup : GroupBase, FixSource<T> {
       for (size_t k = 0; k < pls.size(); k++) {
         dkt_plan *pl = pls[k];
         const size_t ri = c * pls.size() + k;
-        lds = std::max(lds, lds_of(pl, nq));
+        lds = std::max(lds, lds_of(pl));
         ConfArgs &A = hp[ri].A;
         A.tiles = pl->ctiles.p;
         A.tile_nodes = pl->tile_nodes.p;

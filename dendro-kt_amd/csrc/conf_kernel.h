@@ -64,28 +64,37 @@ constexpr int kMaxConfWeights = 256;
 // number of 32-bit words; even nPe keep the level in leaf_lev.
 __host__ __device__ constexpr int conf_row(int npe) { return npe % 2 ? npe + 1 : npe; }
 
-// One tile of one plan (the workgroup may have more work-items than the
-// plan's tile_leaves; they idle in the element phases and help in the loops).
+// Item `item` of one plan: column item % nq of tile item / nq, so that a tile's
+// columns run next to each other and share its maps in L2 (the workgroup may
+// have more work-items than the plan's tile_leaves; they idle in the element
+// phases and help in the loops).  Eight FP64 columns on the 3D p = 2 mesh of 8.9M
+// nodes: 3929 us with a column loop in the workgroup and the LDS of all columns,
+// 1865 so; two columns 505 and 406.
 // CAP: per-level captured element matrices (DKT_OP_CAPTURED), kref pointing
 // to [level][nPe][nPe]; a separate instantiation, since the dense product's
 // registers would otherwise count against the closed-form operators too.
 template <typename T, int DIM, int P, bool CAP = false>
-__device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int tile, const T *__restrict__ kref,
+__device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int item, const T *__restrict__ kref,
                                               const T *__restrict__ term_w, const T *__restrict__ x,
                                               T *__restrict__ y, T *__restrict__ partial) {
   constexpr int NPE = Pow<P + 1, DIM>::v;
   extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int nq = A.nq, tile = nq == 1 ? item : item / nq;
+  {
+    const int q = item - tile * nq;
+    x += q;
+    y += q;
+    partial += q;
+  }
   const ConfTileHdr th = A.tiles[tile];
-  const int nq = A.nq;
   size_t off = 0;
   auto carve = [&](size_t bytes) {
     unsigned char *p = smem_raw + off;
     off += (bytes + 15) & ~(size_t)15;
     return p;
   };
-  T *x_loc = reinterpret_cast<T *>(carve((size_t)A.max_points * nq * sizeof(T)));
-  // One column: the accumulator reuses x_loc once every element has read it.
-  T *y_loc = nq == 1 ? x_loc : reinterpret_cast<T *>(carve((size_t)A.max_points * nq * sizeof(T)));
+  T *x_loc = reinterpret_cast<T *>(carve((size_t)A.max_points * sizeof(T)));
+  T *y_loc = x_loc;  // the accumulator, once every element has read x_loc
   T *wt = reinterpret_cast<T *>(carve((size_t)A.nw * sizeof(T)));  // the weight table
   const int tid = threadIdx.x, nthr = blockDim.x;
   // The weight table's first batch, loaded with the stage loads and stored after them.
@@ -116,8 +125,8 @@ __device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int tile, cons
   const int npts = th.nnode + th.nv;
   // Staging in batches of kCB per work-item: every load of a batch is issued
   // before any of its values is used, so a batch costs one memory round trip
-  // after its node ids, not kCB.  The first column's values are loaded before
-  // the Dirichlet flags, and the flags unconditionally (entries past the
+  // after its node ids, not kCB.  The values are loaded before the
+  // Dirichlet flags, and the flags unconditionally (entries past the
   // tile's nodes read node 0's): a flag tested inside a per-entry branch is
   // waited for there, one round trip per entry.
   constexpr int kCB = 4;
@@ -137,19 +146,12 @@ __device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int tile, cons
     if (A.dir_in)
 #pragma unroll
       for (int b = 0; b < kCB; b++) d[b] = A.dir_in[g[b] >= 0 ? g[b] : 0];
-    for (int q = 0; q < nq; q++) {
-      if (q > 0)
 #pragma unroll
-        for (int b = 0; b < kCB; b++) xv[b] = g[b] >= 0 ? x[(size_t)g[b] * A.ld + q] : T(0);
-#pragma unroll
-      for (int b = 0; b < kCB; b++)
-        if (g[b] >= 0) x_loc[(j0 + b * nthr) * nq + q] = d[b] ? T(0) : xv[b];
-    }
+    for (int b = 0; b < kCB; b++)
+      if (g[b] >= 0) x_loc[j0 + b * nthr] = d[b] ? T(0) : xv[b];
   }
   if (tid < A.nw) wt[tid] = w_first;
   for (int i = tid + nthr; i < A.nw; i += nthr) wt[i] = term_w[i];
-  if (nq > 1)
-    for (int j = tid; j < npts * nq; j += nthr) y_loc[j] = T(0);
   __syncthreads();
   // Hanging point values: each row over the staged nodes, terms in row order,
   // read kTB at a time with all loads of a batch issued together.  Entries
@@ -162,76 +164,70 @@ __device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int tile, cons
   const uint32_t *tpk = A.term_pk + th.t0;
   for (int v = tid; v < th.nv; v += nthr) {
     const int k0 = A.virt_off[th.v0 + v], k1 = v + 1 < th.nv ? A.virt_off[th.v0 + v + 1] : th.nt;
-    for (int q = 0; q < nq; q++) {
-      T s = T(0);
-      for (int k = k0; k < k1; k += kTB) {
-        uint32_t e[kTB];
+    T s = T(0);
+    for (int k = k0; k < k1; k += kTB) {
+      uint32_t e[kTB];
 #pragma unroll
-        for (int b = 0; b < kTB; b++) e[b] = tpk[min(k + b, k1 - 1)];
+      for (int b = 0; b < kTB; b++) e[b] = tpk[min(k + b, k1 - 1)];
 #pragma unroll
-        for (int b = 0; b < kTB; b++) {
-          const T xv = x_loc[(int)(e[b] & 0xFFFFu) * nq + q];
-          s += wt[e[b] >> 16] * (k + b < k1 ? xv : T(0));
-        }
+      for (int b = 0; b < kTB; b++) {
+        const T xv = x_loc[e[b] & 0xFFFFu];
+        s += wt[e[b] >> 16] * (k + b < k1 ? xv : T(0));
       }
-      x_loc[(th.nnode + v) * nq + q] = s;
     }
+    x_loc[th.nnode + v] = s;
   }
   __syncthreads();
   const T scale = (T)ldexp(1.0, -level_of() * A.hp);
 
   // 2. Elements.
-  for (int q = 0; q < nq; q++) {
-    T v[NPE];
-    if (active) {
-      T u[NPE];
+  T v[NPE];
+  if (active) {
+    T u[NPE];
 #pragma unroll
-      for (int r = 0; r < NPE; r++) u[r] = x_loc[loc_of(r) * nq + q];
-      if constexpr (CAP) {
-        // Per-level element matrices (row-major, v = K u; the level carries
-        // the element size, so no scale): the lanes of a wavefront mostly
-        // share a level, so each entry is one broadcast load.
-        const T *K = kref + (size_t)level_of() * NPE * NPE;
+    for (int r = 0; r < NPE; r++) u[r] = x_loc[loc_of(r)];
+    if constexpr (CAP) {
+      // Per-level element matrices (row-major, v = K u; the level carries
+      // the element size, so no scale): the lanes of a wavefront mostly
+      // share a level, so each entry is one broadcast load.
+      const T *K = kref + (size_t)level_of() * NPE * NPE;
 #pragma unroll
-        for (int i = 0; i < NPE; i++) {
-          T acc = T(0);
+      for (int i = 0; i < NPE; i++) {
+        T acc = T(0);
 #pragma unroll
-          for (int j = 0; j < NPE; j++) acc += K[i * NPE + j] * u[j];
-          v[i] = acc;
-        }
-      } else if constexpr (P == 1) {
-        if (A.op == 0)
-          q1_apply<T, DIM, 0>(u, v, scale);
-        else if (A.op == 1)
-          q1_apply<T, DIM, 1>(u, v, scale);
-        else
-#pragma unroll
-          for (int i = 0; i < NPE; i++) v[i] = scale * u[i];
-      } else {
-        // The element scale 2^(-level hp) as an exponent (one register, not
-        // an FP64 pair); scaling by a power of two gives the same bits in any
-        // position.
-        q2_apply<T, DIM>(u, kref, A.op, T(1));
-        if constexpr (LEV_IN_ROW) asm volatile("" : "+v"(lw[NW - 1]));  // the level is read here, not kept
-        const int ex = -level_of() * A.hp;
-#pragma unroll
-        for (int i = 0; i < NPE; i++) v[i] = ldexp(u[i], ex);
+        for (int j = 0; j < NPE; j++) acc += K[i * NPE + j] * u[j];
+        v[i] = acc;
       }
-    }
-    // The packed indices are opaque from here on, so the rank phases unpack
-    // them again instead of keeping the gather's unpacked copies alive.
+    } else if constexpr (P == 1) {
+      if (A.op == 0)
+        q1_apply<T, DIM, 0>(u, v, scale);
+      else if (A.op == 1)
+        q1_apply<T, DIM, 1>(u, v, scale);
+      else
 #pragma unroll
-    for (int w = 0; w < NW; w++) asm volatile("" : "+v"(lw[w]));
-    if (nq == 1) {
-      __syncthreads();
-      for (int j = tid; j < npts; j += nthr) y_loc[j] = T(0);
-      __syncthreads();
-    }
+        for (int i = 0; i < NPE; i++) v[i] = scale * u[i];
+    } else {
+      // The element scale 2^(-level hp) as an exponent (one register, not
+      // an FP64 pair); scaling by a power of two gives the same bits in any
+      // position.
+      q2_apply<T, DIM>(u, kref, A.op, T(1));
+      if constexpr (LEV_IN_ROW) asm volatile("" : "+v"(lw[NW - 1]));  // the level is read here, not kept
+      const int ex = -level_of() * A.hp;
 #pragma unroll
-    for (int r = 0; r < NPE; r++) {
-      if (active) y_loc[loc_of(r) * nq + q] += v[r];
-      __syncthreads();
+      for (int i = 0; i < NPE; i++) v[i] = ldexp(u[i], ex);
     }
+  }
+  // The packed indices are opaque from here on, so the rank phases unpack
+  // them again instead of keeping the gather's unpacked copies alive.
+#pragma unroll
+  for (int w = 0; w < NW; w++) asm volatile("" : "+v"(lw[w]));
+  __syncthreads();
+  for (int j = tid; j < npts; j += nthr) y_loc[j] = T(0);
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < NPE; r++) {
+    if (active) y_loc[loc_of(r)] += v[r];
+    __syncthreads();
   }
 
   // 3. Transposed rows: per node, its terms in sorted order (one segment per node).
@@ -240,20 +236,18 @@ __device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int tile, cons
     const uint32_t sg = A.seg[th.s0 + g];
     const int j = (int)(sg & 0xFFFFu), m0 = (int)(sg >> 16);
     const int m1 = g + 1 < th.ns ? (int)(A.seg[th.s0 + g + 1] >> 16) : th.nt;
-    for (int q = 0; q < nq; q++) {
-      T acc = T(0);
-      for (int m = m0; m < m1; m += kTB) {
-        uint32_t e[kTB];
+    T acc = T(0);
+    for (int m = m0; m < m1; m += kTB) {
+      uint32_t e[kTB];
 #pragma unroll
-        for (int b = 0; b < kTB; b++) e[b] = spk[min(m + b, m1 - 1)];
+      for (int b = 0; b < kTB; b++) e[b] = spk[min(m + b, m1 - 1)];
 #pragma unroll
-        for (int b = 0; b < kTB; b++) {  // padding adds an exact +-0, as in the rows
-          const T yv = y_loc[(th.nnode + (int)(e[b] & 0xFFFFu)) * nq + q];
-          acc += wt[e[b] >> 16] * (m + b < m1 ? yv : T(0));
-        }
+      for (int b = 0; b < kTB; b++) {  // padding adds an exact +-0, as in the rows
+        const T yv = y_loc[th.nnode + (int)(e[b] & 0xFFFFu)];
+        acc += wt[e[b] >> 16] * (m + b < m1 ? yv : T(0));
       }
-      y_loc[j * nq + q] += acc;
     }
+    y_loc[j] += acc;
   }
   __syncthreads();
 
@@ -275,11 +269,10 @@ __device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int tile, cons
     for (int b = 0; b < kCB; b++) {
       const int j = j0 + b * nthr;
       if (o[b] == INT32_MIN) continue;
-      if (o[b] >= 0) {
-        for (int q = 0; q < nq; q++) y[(size_t)o[b] * A.ld + q] = d[b] ? T(0) : y_loc[j * nq + q];
-      } else {
-        for (int q = 0; q < nq; q++) partial[(size_t)(-o[b] - 1) * nq + q] = y_loc[j * nq + q];
-      }
+      if (o[b] >= 0)
+        y[(size_t)o[b] * A.ld] = d[b] ? T(0) : y_loc[j];
+      else
+        partial[(size_t)(-o[b] - 1) * nq] = y_loc[j];
     }
   }
 }
@@ -293,11 +286,11 @@ __global__ void __launch_bounds__(kTileThreads) conf_tile_kernel(ConfArgs A, con
   conf_tile_body<T, DIM, P, CAP>(A, xcd_tile(blockIdx.x, gridDim.x), kref, term_w, x, y, partial);
 }
 
-// LDS bytes of conf_tile_kernel for nq right-hand sides and a weight table of nw entries.
+// LDS bytes of conf_tile_kernel with a weight table of nw entries.
 template <typename T, int NPE>
-inline size_t conf_lds_bytes(int max_points, int nq, int nw) {
+inline size_t conf_lds_bytes(int max_points, int nw) {
   auto r16 = [](size_t b) { return (b + 15) & ~(size_t)15; };
-  return (nq == 1 ? 1 : 2) * r16((size_t)max_points * nq * sizeof(T)) + r16((size_t)nw * sizeof(T));
+  return r16((size_t)max_points * sizeof(T)) + r16((size_t)nw * sizeof(T));
 }
 
 }  // namespace dkt

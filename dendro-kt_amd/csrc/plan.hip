@@ -835,7 +835,7 @@ TiledHost build_tiled_host(const MeshParams &mp, const Traversal &tr, size_t N, 
 
 template <int NPE>
 size_t lds_f64(const TiledHost &o, int T) {
-  return tile_lds_bytes<double, NPE>(TileDims{o.max_nodes, o.max_grp, o.max_he, o.max_rd, o.max_cr, T, o.max_hang}, 1);
+  return tile_lds_bytes<double, NPE>(TileDims{o.max_nodes, o.max_grp, o.max_he, o.max_rd, o.max_cr, T, o.max_hang});
 }
 
 void build_tiled(dkt_plan *pl, const MeshParams &mp, const Traversal &tr, int requested) {
@@ -1210,7 +1210,7 @@ void build_conf_tiled(dkt_plan *pl, const MeshParams &mp, const Traversal &tr, i
     ConfTileOut().nodes.swap(to.nodes);  // release as we go
   }
   // Halve the tiles while one right-hand side in FP64 does not fit in LDS.
-  pl->lds_bytes = conf_lds_bytes<double, 4>(max_points, 1, (int)wtab.size());
+  pl->lds_bytes = conf_lds_bytes<double, 4>(max_points, (int)wtab.size());
   if (pl->lds_bytes > (size_t)kLdsLimit && T > 16) return build_conf_tiled(pl, mp, tr, T / 2);
   // Owned nodes go to y; a node in several tiles gets a partial slot per tile
   // (node-major, tile order), summed by fixup_kernel.
@@ -1303,6 +1303,19 @@ void run_simple(dkt_plan *pl, int nrhs, const T *x, T *y, int mask, hipStream_t 
   HIP_OK(hipGetLastError());
 }
 
+// Columns of one launch, as separate workgroups: kCols, which bounds the
+// partial sums (a tile's columns run next to each other, so more columns in a
+// launch gain nothing), or as many as fit in the caller's scratch.
+constexpr int kCols = 8;
+
+template <typename T>
+int launch_columns(const dkt_plan *pl, int nrhs, const ExtScratch *ext) {
+  int chunk = std::min(nrhs, kCols);
+  while (ext && chunk > 1 && pl->npartial * (size_t)chunk * sizeof(T) > ext->bytes) chunk--;
+  if (pl->ntiles * (size_t)chunk > (size_t)INT32_MAX) throw std::invalid_argument("too many tiles and columns");
+  return chunk;
+}
+
 template <typename T, int DIM, int P>
 void run_tiled(dkt_plan *pl, int nrhs, const T *x, T *y, int mask, hipStream_t st, const int *cancel,
                const ExtScratch *ext) {
@@ -1311,14 +1324,10 @@ void run_tiled(dkt_plan *pl, int nrhs, const T *x, T *y, int mask, hipStream_t s
   const T *kmat = P == 2 ? (f64 ? (const T *)pl->kfac64.p : (const T *)pl->kfac32.p)
                          : (f64 ? (const T *)pl->kmat64.p : (const T *)pl->kmat32.p);
   const T *cw = f64 ? (const T *)pl->carry_w64.p : (const T *)pl->carry_w32.p;
-  auto lds_for = [&](int nq) {
-    return tile_lds_bytes<T, NPE>(
-        TileDims{pl->max_nodes, pl->max_grp, pl->max_he, pl->max_rd, pl->max_cr, pl->tile_leaves, pl->max_hang}, nq);
-  };
-  // Columns are processed in chunks whose LDS footprint stays within budget.
-  if (lds_for(1) > kLdsLimit) throw std::invalid_argument("tile does not fit in LDS");
-  int chunk = 1;
-  while (chunk < nrhs && lds_for(chunk + 1) <= kLdsLimit) chunk++;
+  const TileDims dims{pl->max_nodes, pl->max_grp, pl->max_he, pl->max_rd, pl->max_cr, pl->tile_leaves, pl->max_hang};
+  const size_t lds = tile_lds_bytes<T, NPE>(dims);
+  if (lds > kLdsLimit) throw std::invalid_argument("tile does not fit in LDS");
+  const int chunk = launch_columns<T>(pl, nrhs, ext);
   T *part = matvec_scratch<T>(pl, std::max<size_t>(1, pl->npartial * (size_t)chunk), ext);
   TileArgs A;
   A.tiles = pl->tiles.p;
@@ -1337,18 +1346,15 @@ void run_tiled(dkt_plan *pl, int nrhs, const T *x, T *y, int mask, hipStream_t s
   A.hp = pl->hp;
   A.ld = nrhs;
   A.blocks = pl->blocks.p;
-  A.dims = TileDims{pl->max_nodes, pl->max_grp, pl->max_he, pl->max_rd, pl->max_cr, pl->tile_leaves, pl->max_hang};
+  A.dims = dims;
   for (int q0 = 0; q0 < nrhs; q0 += chunk) {
     const int nq = std::min(chunk, nrhs - q0);
     A.nq = nq;
     if (pl->profiling && !ext) HIP_OK(hipEventRecord(pl->next_event(), st));
     if (pl->ntiles) {
-      if (nq == 1)
-        hipLaunchKernelGGL((tile_kernel<T, DIM, P, true>), dim3(pl->ntiles), dim3(pl->tile_leaves), lds_for(nq), st, A,
-                           kmat, cw, x + q0, y + q0, part);
-      else
-        hipLaunchKernelGGL((tile_kernel<T, DIM, P, false>), dim3(pl->ntiles), dim3(pl->tile_leaves), lds_for(nq), st,
-                           A, kmat, cw, x + q0, y + q0, part);
+      auto kernel = nq == 1 ? tile_kernel<T, DIM, P, true> : tile_kernel<T, DIM, P, false>;
+      hipLaunchKernelGGL(kernel, dim3(pl->ntiles * nq), dim3(pl->tile_leaves), lds, st, A, kmat, cw, x + q0, y + q0,
+                         part);
       HIP_OK(hipGetLastError());
     }
     if (pl->profiling && !ext) HIP_OK(hipEventRecord(pl->next_event(), st));
@@ -1362,23 +1368,16 @@ void run_tiled(dkt_plan *pl, int nrhs, const T *x, T *y, int mask, hipStream_t s
   }
 }
 
-// Columns of one launch over point tiles: kPointCols, which bounds the partial
-// sums (a column's tiles run next to each other, so more columns in a launch
-// gain nothing), or as many as fit in the caller's scratch.
-constexpr int kPointCols = 8;
-
 template <typename T, int DIM>
 void run_points(dkt_plan *pl, int nrhs, const T *x, T *y, int mask, hipStream_t st, const int *cancel,
                 const ExtScratch *ext) {
   const bool f64 = sizeof(T) == 8;
   const T *kmat = f64 ? (const T *)pl->kmat64.p : (const T *)pl->kmat32.p;
-  int chunk = std::min(nrhs, kPointCols);
-  while (ext && chunk > 1 && pl->npartial * (size_t)chunk * sizeof(T) > ext->bytes) chunk--;
+  const int chunk = launch_columns<T>(pl, nrhs, ext);
   T *part = matvec_scratch<T>(pl, std::max<size_t>(1, pl->npartial * (size_t)chunk), ext);
   for (int q0 = 0; q0 < nrhs; q0 += chunk) {
     const int nq = std::min(chunk, nrhs - q0);
     const PtArgs A = pl->point_args(mask, cancel, nq, nrhs);
-    if (pl->ntiles * (size_t)nq > (size_t)INT32_MAX) throw std::invalid_argument("too many tiles and columns");
     if (pl->profiling && !ext) HIP_OK(hipEventRecord(pl->next_event(), st));
     if (pl->ntiles) {
       auto kernel = pl->per_level ? point_kernel<T, DIM, true> : point_kernel<T, DIM, false>;
@@ -1404,10 +1403,9 @@ void run_conf(dkt_plan *pl, int nrhs, const T *x, T *y, int mask, hipStream_t st
   const T *kmat = P == 2 && !pl->per_level ? (f64 ? (const T *)pl->kfac64.p : (const T *)pl->kfac32.p)
                                            : (f64 ? (const T *)pl->kmat64.p : (const T *)pl->kmat32.p);
   const T *tw = f64 ? (const T *)pl->term_w64.p : (const T *)pl->term_w32.p;
-  auto lds_for = [&](int nq) { return conf_lds_bytes<T, NPE>(pl->max_nodes, nq, pl->nw); };
-  if (lds_for(1) > kLdsLimit) throw std::invalid_argument("tile does not fit in LDS");
-  int chunk = 1;
-  while (chunk < nrhs && lds_for(chunk + 1) <= kLdsLimit) chunk++;
+  const size_t lds = conf_lds_bytes<T, NPE>(pl->max_nodes, pl->nw);
+  if (lds > kLdsLimit) throw std::invalid_argument("tile does not fit in LDS");
+  const int chunk = launch_columns<T>(pl, nrhs, ext);
   T *part = matvec_scratch<T>(pl, std::max<size_t>(1, pl->npartial * (size_t)chunk), ext);
   ConfArgs A;
   A.tiles = pl->ctiles.p;
@@ -1433,12 +1431,9 @@ void run_conf(dkt_plan *pl, int nrhs, const T *x, T *y, int mask, hipStream_t st
     A.nq = nq;
     if (pl->profiling && !ext) HIP_OK(hipEventRecord(pl->next_event(), st));
     if (pl->ntiles) {
-      if (pl->per_level)
-        hipLaunchKernelGGL((conf_tile_kernel<T, DIM, P, true>), dim3(pl->ntiles), dim3(pl->tile_leaves), lds_for(nq),
-                           st, A, kmat, tw, x + q0, y + q0, part);
-      else
-        hipLaunchKernelGGL((conf_tile_kernel<T, DIM, P, false>), dim3(pl->ntiles), dim3(pl->tile_leaves),
-                           lds_for(nq), st, A, kmat, tw, x + q0, y + q0, part);
+      auto kernel = pl->per_level ? conf_tile_kernel<T, DIM, P, true> : conf_tile_kernel<T, DIM, P, false>;
+      hipLaunchKernelGGL(kernel, dim3(pl->ntiles * nq), dim3(pl->tile_leaves), lds, st, A, kmat, tw, x + q0, y + q0,
+                         part);
       HIP_OK(hipGetLastError());
     }
     if (pl->profiling && !ext) HIP_OK(hipEventRecord(pl->next_event(), st));

@@ -70,12 +70,12 @@ struct Group {
   static constexpr int v = NPE <= 4 ? 4 : (NPE <= 8 ? 8 : (NPE <= 16 ? 16 : 32));
 };
 
-// Elements of the tile kernel's y_loc: the accumulator, and with one column
-// (the single-column kernel) the groups' parent values before it.
+// Elements of the tile kernel's y_loc: the groups' parent values, then the
+// accumulator.
 template <int NPE>
-__host__ __device__ inline size_t tile_yloc_elems(const TileDims &D, int nq) {
-  const size_t acc = (size_t)D.max_nodes * nq, par = (size_t)D.max_grp * NPE;
-  return nq == 1 && par > acc ? par : acc;
+__host__ __device__ inline size_t tile_yloc_elems(const TileDims &D) {
+  const size_t acc = (size_t)D.max_nodes, par = (size_t)D.max_grp * NPE;
+  return par > acc ? par : acc;
 }
 
 // Bytes of the tile kernel's shared LDS region: reader values or per-group
@@ -147,20 +147,33 @@ __device__ __forceinline__ T interp_lanes(T a, int lane, int c) {
   return a;
 }
 
-// One tile of one plan (the workgroup may have more work-items than the
-// plan's tile_leaves; they idle in the leaf phases and help in the loops).
-// ONE: a single right-hand side per launch (nq = 1 at compile time, which
-// keeps the leaf state out of a runtime column loop and halves the VGPRs).
+// Item `item` of one plan: column item % nq of tile item / nq, so that the
+// columns of a tile run next to each other and share its maps and the lines of
+// the node-major vectors in L2 (the workgroup may have more work-items than the
+// plan's tile_leaves; they idle in the leaf phases and help in the loops).  A
+// column loop inside the workgroup held the LDS of all columns, which left few
+// workgroups on a CU: eight FP32 columns on 82,776 3D p = 2 elements took 193 us
+// against 81, eight FP64 ones on the 4D tree of 2M points 23.8 ms against 9.5.
+// ONE: a single column, item = tile; carrying a column index there cost that 4D
+// matvec 1 % in FP64 and 4 % in FP32 (612 to 635 us).
 template <typename T, int DIM, int P, bool ONE>
-__device__ __forceinline__ void tile_body(const TileArgs &A, int tile, const T *__restrict__ kref,
+__device__ __forceinline__ void tile_body(const TileArgs &A, int item, const T *__restrict__ kref,
                                          const T *__restrict__ carry_w, const T *__restrict__ x, T *__restrict__ y,
                                          T *__restrict__ partial) {
   constexpr int NPE = Pow<P + 1, DIM>::v;
   constexpr int G = Group<NPE>::v;
   extern __shared__ __align__(16) unsigned char smem_raw[];
+  int tile = item;
+  const int nq = ONE ? 1 : A.nq;
+  if constexpr (!ONE) {
+    tile = item / nq;
+    const int q = item - tile * nq;
+    x += q;
+    y += q;
+    partial += q;
+  }
   const TileHdr th = A.tiles[tile];
   const TileDims D = A.dims;
-  const int nq = ONE ? 1 : A.nq;
   const int TL = D.tile_leaves;
   size_t off = 0;
   auto carve = [&](size_t bytes) {
@@ -168,15 +181,15 @@ __device__ __forceinline__ void tile_body(const TileArgs &A, int tile, const T *
     off += (bytes + 15) & ~(size_t)15;
     return p;
   };
-  T *x_loc = reinterpret_cast<T *>(carve((size_t)D.max_nodes * nq * sizeof(T)));
-  // ONE: y_loc first holds the parent values of the sibling groups [group][slot]
+  T *x_loc = reinterpret_cast<T *>(carve((size_t)D.max_nodes * sizeof(T)));
+  // y_loc first holds the parent values of the sibling groups [group][slot]
   // (replay and element phases), then the accumulator.
-  T *y_loc = reinterpret_cast<T *>(carve(tile_yloc_elems<NPE>(D, nq) * sizeof(T)));
+  T *y_loc = reinterpret_cast<T *>(carve(tile_yloc_elems<NPE>(D) * sizeof(T)));
   T *pval = y_loc;
   // Shared region: reader values [reader][slot] (replay to element phase),
   // then group sums [group][slot] (transposed phase).
   T *ubuf = reinterpret_cast<T *>(carve(tile_region_bytes<T, NPE>(D)));
-  T *cst = reinterpret_cast<T *>(carve((size_t)NPE * nq * sizeof(T)));  // parent buffer at the tile start
+  T *cst = reinterpret_cast<T *>(carve((size_t)NPE * sizeof(T)));  // parent buffer at the tile start
   uint32_t *hent = reinterpret_cast<uint32_t *>(carve((size_t)D.max_he * 4));
   uint32_t *cw_s = reinterpret_cast<uint32_t *>(carve((size_t)(D.max_hang + 1) * 4));  // chain word per hanging index
   uint16_t *gploc = reinterpret_cast<uint16_t *>(carve((size_t)D.max_grp * NPE * 2));
@@ -239,19 +252,9 @@ __device__ __forceinline__ void tile_body(const TileArgs &A, int tile, const T *
     if (A.dir_in)
 #pragma unroll
       for (int b = 0; b < kNB; b++) d[b] = A.dir_in[g[b] >= 0 ? g[b] : 0];
-    for (int q = 0; q < nq; q++) {
-      if (q > 0)
 #pragma unroll
-        for (int b = 0; b < kNB; b++) xv[b] = g[b] >= 0 ? x[(size_t)g[b] * A.ld + q] : T(0);
-#pragma unroll
-      for (int b = 0; b < kNB; b++) {
-        const int j = j0 + b * nthr;
-        if (g[b] >= 0) {
-          x_loc[j * nq + q] = d[b] ? T(0) : xv[b];
-          if constexpr (!ONE) y_loc[j * nq + q] = T(0);
-        }
-      }
-    }
+    for (int b = 0; b < kNB; b++)
+      if (g[b] >= 0) x_loc[j0 + b * nthr] = d[b] ? T(0) : xv[b];
   }
 #pragma unroll
   for (int b = 0; b < 2; b++) {
@@ -271,7 +274,7 @@ __device__ __forceinline__ void tile_body(const TileArgs &A, int tile, const T *
   if (hang) cw_s[hidx] = (uint32_t)child | ((uint32_t)grp_id << 8);
   __syncthreads();
 
-  // 2. Parent-buffer state at the tile start, every column: slot s sums its
+  // 2. Parent-buffer state at the tile start: slot s sums its
   //    terms (a header of slot offsets, then the terms by slot) in plan order,
   //    read kNB at a time with all loads of a batch issued together.  Entries
   //    past the slot's last term repeat it with the value 0: an exact +-0
@@ -281,30 +284,26 @@ __device__ __forceinline__ void tile_body(const TileArgs &A, int tile, const T *
     const uint32_t *ck = A.carry_key + th.cr0;
     const T *cwp = carry_w + th.cr0;
     const int lo = th.ncr > 0 ? (int)ck[tid] : 0, hi = th.ncr > 0 ? (int)ck[tid + 1] : 0;
-    for (int q = 0; q < nq; q++) {
-      T acc = T(0);
-      for (int c = lo; c < hi; c += kNB) {
-        uint32_t kk[kNB];
-        T cwv[kNB];
+    T acc = T(0);
+    for (int c = lo; c < hi; c += kNB) {
+      uint32_t kk[kNB];
+      T cwv[kNB];
 #pragma unroll
-        for (int b = 0; b < kNB; b++) {
-          const int cc = min(c + b, hi - 1);
-          kk[b] = ck[cc];
-          cwv[b] = cwp[cc];
-        }
-#pragma unroll
-        for (int b = 0; b < kNB; b++) {
-          const T xv = x_loc[(kk[b] & 0xFFFFu) * nq + q];
-          acc += cwv[b] * (c + b < hi ? xv : T(0));
-        }
+      for (int b = 0; b < kNB; b++) {
+        const int cc = min(c + b, hi - 1);
+        kk[b] = ck[cc];
+        cwv[b] = cwp[cc];
       }
-      cst[tid * nq + q] = acc;
+#pragma unroll
+      for (int b = 0; b < kNB; b++) {
+        const T xv = x_loc[kk[b] & 0xFFFFu];
+        acc += cwv[b] * (c + b < hi ? xv : T(0));
+      }
     }
+    cst[tid] = acc;
   }
-  if constexpr (ONE)
-    for (int k = tid; k < th.ngrp * NPE; k += nthr) pval[k] = gploc[k] != kNone ? x_loc[gploc[k]] : T(0);
+  for (int k = tid; k < th.ngrp * NPE; k += nthr) pval[k] = gploc[k] != kNone ? x_loc[gploc[k]] : T(0);
   __syncthreads();
-  const uint16_t *ploc = gploc + (size_t)grp_id * NPE;
   const int lane = tid % G, grp = tid / G, ngroups = nthr / G;
   const int sl = lane < NPE ? lane : 0;
   const int wl = tid & 63;  // lane in the wavefront
@@ -314,161 +313,149 @@ __device__ __forceinline__ void tile_body(const TileArgs &A, int tile, const T *
   const uint64_t later = wl == 63 ? 0 : (starts >> (wl + 1));
   const int run_end = later ? wl + 1 + __builtin_ctzll(later) : 64;
 
-  for (int q = 0; q < nq; q++) {
-    // 3. Stale parent-buffer reads: a lane group per replay block runs the
-    //    recurrence over the block's hanging leaves, B_k = W_ck (parent nodes
-    //    where present, else B_(k-1)), and stores B_k of each reader it passes.
-    for (int b0 = 0; b0 < th.nbk; b0 += ngroups) {
-      const int bi = b0 + grp;
-      if (bi >= th.nbk) continue;
-      const uint64_t blk = b0 == 0 ? blk_first : A.blocks[th.bk0 + bi];
-      const int S = (int)(blk & 0xFFFFu), E = (int)((blk >> 16) & 0xFFFFu);
-      int p = (int)((blk >> 32) & 0xFFFFu);
-      const int pend = p + (int)(blk >> 48);
-      int nxt = rdl_s[p] & 255;
-      // Parent value of this lane's slot for hanging index k (kNone: absent).
-      auto parent = [&](uint32_t cw, T &xp) {
-        const size_t gi = (size_t)(cw >> 8) * NPE + sl;
-        const uint16_t pl = gploc[gi];
-        if constexpr (ONE)
-          xp = lane < NPE ? pval[gi] : T(0);
-        else
-          xp = (lane < NPE && pl != kNone) ? x_loc[pl * nq + q] : T(0);
-        return lane < NPE && pl == kNone;
-      };
-      T B;
-      int k;
-      if (S == 0xFFFF) {
-        B = cst[sl * nq + q];
-        k = 0;
-      } else {
-        const uint32_t cw0 = cw_s[S];
-        T xp;
-        parent(cw0, xp);
-        B = interp_lanes<T, DIM, P>(xp, lane, (int)(cw0 & 255u));
-        k = S + 1;
-      }
-      // Chain words and parent values do not depend on B: loaded one step ahead.
-      uint32_t cw = cw_s[k];
+  // 3. Stale parent-buffer reads: a lane group per replay block runs the
+  //    recurrence over the block's hanging leaves, B_k = W_ck (parent nodes
+  //    where present, else B_(k-1)), and stores B_k of each reader it passes.
+  for (int b0 = 0; b0 < th.nbk; b0 += ngroups) {
+    const int bi = b0 + grp;
+    if (bi >= th.nbk) continue;
+    const uint64_t blk = b0 == 0 ? blk_first : A.blocks[th.bk0 + bi];
+    const int S = (int)(blk & 0xFFFFu), E = (int)((blk >> 16) & 0xFFFFu);
+    int p = (int)((blk >> 32) & 0xFFFFu);
+    const int pend = p + (int)(blk >> 48);
+    int nxt = rdl_s[p] & 255;
+    // Parent value of this lane's slot for hanging index k (kNone: absent).
+    auto parent = [&](uint32_t cw, T &xp) {
+      const size_t gi = (size_t)(cw >> 8) * NPE + sl;
+      const uint16_t pl = gploc[gi];
+      xp = lane < NPE ? pval[gi] : T(0);
+      return lane < NPE && pl == kNone;
+    };
+    T B;
+    int k;
+    if (S == 0xFFFF) {
+      B = cst[sl];
+      k = 0;
+    } else {
+      const uint32_t cw0 = cw_s[S];
       T xp;
-      bool ab = parent(cw, xp);
-      for (;; k++) {
-        const bool last = k >= E;
-        const uint32_t cwn = last ? cw : cw_s[k + 1];
-        T xpn;
-        const bool abn = parent(cwn, xpn);
-        B = interp_lanes<T, DIM, P>(ab ? B : xp, lane, (int)(cw & 255u));
-        if (k == nxt) {
-          if (lane < NPE) ubuf[p * NPE + lane] = B;
-          if (lane == 0) ridx_s[rdl_s[p] >> 8] = (uint16_t)p;
-          p++;
-          nxt = p < pend ? (rdl_s[p] & 255) : -1;
-        }
-        if (last) break;
-        cw = cwn;
-        xp = xpn;
-        ab = abn;
-      }
+      parent(cw0, xp);
+      B = interp_lanes<T, DIM, P>(xp, lane, (int)(cw0 & 255u));
+      k = S + 1;
     }
-    __syncthreads();
-    // 4. Element vector and elemental operator: a hanging leaf's missing ranks
-    //    interpolate its parent nodes (readers: the replayed buffer B_k).
-    T v[NPE];
-    if (active) {
-      // Missing ranks first (zero for a leaf without hanging nodes), then the
-      // present ranks replace them: one LDS read per rank, no branches.
-      T u[NPE];
-      if (hang) {
-        if constexpr (ONE) {
-#pragma unroll
-          for (int s = 0; s < NPE; s++) u[s] = pval[grp_id * NPE + s];
-        } else {
-#pragma unroll
-          for (int s = 0; s < NPE; s++) u[s] = ploc[s] != kNone ? x_loc[ploc[s] * nq + q] : T(0);
-        }
-        interp<T, DIM, P, false>(u, child);
-        const int ri = ridx_s[tid];
-        if (ri != kNone)
-#pragma unroll
-          for (int r = 0; r < NPE; r++) u[r] = ubuf[ri * NPE + r];
-      } else {
-#pragma unroll
-        for (int r = 0; r < NPE; r++) u[r] = T(0);
+    // Chain words and parent values do not depend on B: loaded one step ahead.
+    uint32_t cw = cw_s[k];
+    T xp;
+    bool ab = parent(cw, xp);
+    for (;; k++) {
+      const bool last = k >= E;
+      const uint32_t cwn = last ? cw : cw_s[k + 1];
+      T xpn;
+      const bool abn = parent(cwn, xpn);
+      B = interp_lanes<T, DIM, P>(ab ? B : xp, lane, (int)(cw & 255u));
+      if (k == nxt) {
+        if (lane < NPE) ubuf[p * NPE + lane] = B;
+        if (lane == 0) ridx_s[rdl_s[p] >> 8] = (uint16_t)p;
+        p++;
+        nxt = p < pend ? (rdl_s[p] & 255) : -1;
       }
-#pragma unroll
-      for (int r = 0; r < NPE; r++) {
-        const bool present = loc[r] != kNone;
-        const T xv = x_loc[(present ? loc[r] : 0) * nq + q];
-        u[r] = present ? xv : u[r];
-      }
-      if constexpr (P == 1) {
-        if (A.op == 0)
-          q1_apply<T, DIM, 0>(u, v, scale);
-        else if (A.op == 1)
-          q1_apply<T, DIM, 1>(u, v, scale);
-        else
-#pragma unroll
-          for (int i = 0; i < NPE; i++) v[i] = scale * u[i];
-      } else {
-        q2_apply<T, DIM>(u, kref, A.op, scale);
-#pragma unroll
-        for (int i = 0; i < NPE; i++) v[i] = u[i];
-      }
+      if (last) break;
+      cw = cwn;
+      xp = xpn;
+      ab = abn;
     }
-    if constexpr (ONE) {
-      // parent values are consumed: y_loc becomes the accumulator
-      __syncthreads();
-      for (int j = tid; j < th.nnode; j += nthr) y_loc[j] = T(0);
+  }
+  __syncthreads();
+  // 4. Element vector and elemental operator: a hanging leaf's missing ranks
+  //    interpolate its parent nodes (readers: the replayed buffer B_k).
+  T v[NPE];
+  if (active) {
+    // Missing ranks first (zero for a leaf without hanging nodes), then the
+    // present ranks replace them: one LDS read per rank, no branches.
+    T u[NPE];
+    if (hang) {
+#pragma unroll
+      for (int s = 0; s < NPE; s++) u[s] = pval[grp_id * NPE + s];
+      interp<T, DIM, P, false>(u, child);
+      const int ri = ridx_s[tid];
+      if (ri != kNone)
+#pragma unroll
+        for (int r = 0; r < NPE; r++) u[r] = ubuf[ri * NPE + r];
+    } else {
+#pragma unroll
+      for (int r = 0; r < NPE; r++) u[r] = T(0);
     }
-    // 5. Direct outputs, one phase per rank.
 #pragma unroll
     for (int r = 0; r < NPE; r++) {
-      __syncthreads();
-      if (loc[r] != kNone) y_loc[loc[r] * nq + q] += v[r];
+      const bool present = loc[r] != kNone;
+      const T xv = x_loc[present ? loc[r] : 0];
+      u[r] = present ? xv : u[r];
     }
-    // 6. Transposed interpolation of missing ranks, summed over each sibling
-    //    group inside the wavefront (pairwise, fixed order), then per target
-    //    node over its (group, parent rank) entries sorted by target.
-    if (th.nhe > 0) {
-      if (__ballot(hang)) {  // wavefronts without hanging leaves have no groups
-        T w[NPE];
+    if constexpr (P == 1) {
+      if (A.op == 0)
+        q1_apply<T, DIM, 0>(u, v, scale);
+      else if (A.op == 1)
+        q1_apply<T, DIM, 1>(u, v, scale);
+      else
 #pragma unroll
-        for (int r = 0; r < NPE; r++) w[r] = (hang && loc[r] == kNone) ? v[r] : T(0);
-        interp<T, DIM, P, true>(w, child);
+        for (int i = 0; i < NPE; i++) v[i] = scale * u[i];
+    } else {
+      q2_apply<T, DIM>(u, kref, A.op, scale);
 #pragma unroll
-        for (int s = 0; s < NPE; s++) w[s] = (hang && loc[s] == kNone) ? w[s] : T(0);
-        // Pairwise sums inside rows of 16 lanes with DPP row shifts (lane i
-        // reads lane i + d of its row; a 0/1 factor keeps the run), then a run
-        // that continues into the next row adds that row's first partial (a
-        // group spans at most two rows).
-        group_step<T, 0x101, 1>(w, wl, run_end);
-        if constexpr (DIM > 1) group_step<T, 0x102, 2>(w, wl, run_end);
-        if constexpr (DIM > 2) group_step<T, 0x104, 4>(w, wl, run_end);
-        if constexpr (DIM > 3) group_step<T, 0x108, 8>(w, wl, run_end);
-        const int nxt = (wl | 15) + 1;
-        if (__ballot(nxt < run_end)) {
-          const T fx = nxt < run_end ? T(1) : T(0);
+      for (int i = 0; i < NPE; i++) v[i] = u[i];
+    }
+  }
+  // parent values are consumed: y_loc becomes the accumulator
+  __syncthreads();
+  for (int j = tid; j < th.nnode; j += nthr) y_loc[j] = T(0);
+  // 5. Direct outputs, one phase per rank.
 #pragma unroll
-          for (int s = 0; s < NPE; s++) w[s] = fma(__shfl(w[s], nxt & 63, 64), fx, w[s]);
-        }
-        if (hang && aux_ghead(aux))
+  for (int r = 0; r < NPE; r++) {
+    __syncthreads();
+    if (loc[r] != kNone) y_loc[loc[r]] += v[r];
+  }
+  // 6. Transposed interpolation of missing ranks, summed over each sibling
+  //    group inside the wavefront (pairwise, fixed order), then per target
+  //    node over its (group, parent rank) entries sorted by target.
+  if (th.nhe > 0) {
+    if (__ballot(hang)) {  // wavefronts without hanging leaves have no groups
+      T w[NPE];
 #pragma unroll
-          for (int s = 0; s < NPE; s++) ubuf[grp_id * NPE + s] = w[s];
+      for (int r = 0; r < NPE; r++) w[r] = (hang && loc[r] == kNone) ? v[r] : T(0);
+      interp<T, DIM, P, true>(w, child);
+#pragma unroll
+      for (int s = 0; s < NPE; s++) w[s] = (hang && loc[s] == kNone) ? w[s] : T(0);
+      // Pairwise sums inside rows of 16 lanes with DPP row shifts (lane i
+      // reads lane i + d of its row; a 0/1 factor keeps the run), then a run
+      // that continues into the next row adds that row's first partial (a
+      // group spans at most two rows).
+      group_step<T, 0x101, 1>(w, wl, run_end);
+      if constexpr (DIM > 1) group_step<T, 0x102, 2>(w, wl, run_end);
+      if constexpr (DIM > 2) group_step<T, 0x104, 4>(w, wl, run_end);
+      if constexpr (DIM > 3) group_step<T, 0x108, 8>(w, wl, run_end);
+      const int nxt = (wl | 15) + 1;
+      if (__ballot(nxt < run_end)) {
+        const T fx = nxt < run_end ? T(1) : T(0);
+#pragma unroll
+        for (int s = 0; s < NPE; s++) w[s] = fma(__shfl(w[s], nxt & 63, 64), fx, w[s]);
       }
-      __syncthreads();
-      for (int k = tid; k < th.nhe; k += nthr) {
-        const int j = (int)(hent[k] >> 16);
-        if (k > 0 && (int)(hent[k - 1] >> 16) == j) continue;  // not a segment head
-        T acc = T(0);
-        for (int m = k; m < th.nhe && (int)(hent[m] >> 16) == j; m++) {
-          const uint32_t e = hent[m];
-          acc += ubuf[(int)(e & 255u) * NPE + (int)((e >> 8) & 255u)];
-        }
-        y_loc[j * nq + q] += acc;
-      }
+      if (hang && aux_ghead(aux))
+#pragma unroll
+        for (int s = 0; s < NPE; s++) ubuf[grp_id * NPE + s] = w[s];
     }
     __syncthreads();
+    for (int k = tid; k < th.nhe; k += nthr) {
+      const int j = (int)(hent[k] >> 16);
+      if (k > 0 && (int)(hent[k - 1] >> 16) == j) continue;  // not a segment head
+      T acc = T(0);
+      for (int m = k; m < th.nhe && (int)(hent[m] >> 16) == j; m++) {
+        const uint32_t e = hent[m];
+        acc += ubuf[(int)(e & 255u) * NPE + (int)((e >> 8) & 255u)];
+      }
+      y_loc[j] += acc;
+    }
   }
+  __syncthreads();
   // 7. Write out: owned nodes to y, shared nodes to their partial slot.
   for (int j0 = tid; j0 < th.nnode; j0 += kNB * nthr) {
     int o[kNB];
@@ -487,28 +474,26 @@ __device__ __forceinline__ void tile_body(const TileArgs &A, int tile, const T *
     for (int b = 0; b < kNB; b++) {
       const int j = j0 + b * nthr;
       if (o[b] == INT32_MIN) continue;
-      for (int q = 0; q < nq; q++) {
-        const T acc = y_loc[j * nq + q];
-        if (o[b] >= 0)
-          y[(size_t)o[b] * A.ld + q] = d[b] ? T(0) : acc;
-        else
-          partial[(size_t)(-o[b] - 1) * nq + q] = acc;
-      }
+      const T acc = y_loc[j];
+      if (o[b] >= 0)
+        y[(size_t)o[b] * A.ld] = d[b] ? T(0) : acc;
+      else
+        partial[(size_t)(-o[b] - 1) * nq] = acc;
     }
   }
 }
 
 // Waves per SIMD the compiler is asked to fit: 8, the most, for the p = 1
-// single-column kernels whose vector registers allow it (their scalar
+// kernels whose vector registers allow it (their scalar
 // registers, the uniform tile fields, otherwise hold them to 7); 1 leaves the
 // register allocation free.
-template <typename T, int DIM, int P, bool ONE>
+template <typename T, int DIM, int P>
 constexpr int tile_waves() {
-  return ONE && P == 1 && (sizeof(T) == 4 || DIM <= 3) ? 8 : 1;
+  return P == 1 && (sizeof(T) == 4 || DIM <= 3) ? 8 : 1;
 }
 
 template <typename T, int DIM, int P, bool ONE>
-__global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(tile_waves<T, DIM, P, ONE>())))
+__global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(tile_waves<T, DIM, P>())))
 tile_kernel(TileArgs A, const T *__restrict__ kref, const T *__restrict__ carry_w, const T *__restrict__ x,
             T *__restrict__ y, T *__restrict__ partial) {
   if (A.cancel && *A.cancel) return;
@@ -540,10 +525,10 @@ __device__ __forceinline__ int find_range(const int *__restrict__ starts, int n,
   return __builtin_amdgcn_readfirstlane(lo);
 }
 
-// All tiles of a batch of same-(dim, p) plans in one launch: batch tile
-// t = xcd_tile(b) of workgroup b is tile t - tile_start[k] of plan k.
+// All tiles and columns of a batch of same-(dim, p) plans in one launch: batch
+// item t = xcd_tile(b) of workgroup b is item t - tile_start[k] of plan k.
 template <typename T, int DIM, int P, bool ONE>
-__global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(tile_waves<T, DIM, P, ONE>())))
+__global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(tile_waves<T, DIM, P>())))
 tile_kernel_batch(const BatchPlan<T> *__restrict__ plans, const int *__restrict__ tile_start, int nplans) {
   const int t = xcd_tile(blockIdx.x, gridDim.x);
   const int k = find_range(tile_start, nplans, t);
@@ -580,13 +565,13 @@ __global__ void __launch_bounds__(256) fixup_kernel(int ns, const int32_t *__res
   for (int q = 0; q < nq; q++) y[(size_t)n * ld + q] = z ? T(0) : sum_partials(partial, a, b, nq, q);
 }
 
-// LDS bytes of one tile for nq right-hand sides (layout of tile_kernel).
+// LDS bytes of one tile (layout of tile_kernel).
 template <typename T, int NPE>
-inline size_t tile_lds_bytes(const TileDims &D, int nq) {
+inline size_t tile_lds_bytes(const TileDims &D) {
   auto r16 = [](size_t b) { return (b + 15) & ~(size_t)15; };
-  return r16((size_t)D.max_nodes * nq * sizeof(T)) + r16(tile_yloc_elems<NPE>(D, nq) * sizeof(T)) +
+  return r16((size_t)D.max_nodes * sizeof(T)) + r16(tile_yloc_elems<NPE>(D) * sizeof(T)) +
          r16(tile_region_bytes<T, NPE>(D)) +
-         r16((size_t)NPE * nq * sizeof(T)) + r16((size_t)D.max_he * 4) + r16((size_t)(D.max_hang + 1) * 4) +
+         r16((size_t)NPE * sizeof(T)) + r16((size_t)D.max_he * 4) + r16((size_t)(D.max_hang + 1) * 4) +
          r16((size_t)D.max_grp * NPE * 2) + r16((size_t)D.tile_leaves * 2) + r16((size_t)D.max_rd * 2);
 }
 
