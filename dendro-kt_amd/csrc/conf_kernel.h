@@ -224,10 +224,27 @@ __device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int item, cons
   __syncthreads();
   for (int j = tid; j < npts; j += nthr) y_loc[j] = T(0);
   __syncthreads();
+  if constexpr (P == 2) {
+    constexpr RankPhases<DIM> RP;
 #pragma unroll
-  for (int r = 0; r < NPE; r++) {
-    if (active) y_loc[loc_of(r)] += v[r];
-    __syncthreads();
+    for (int ph = 0; ph < RP.n; ph++) {
+      if (active) {
+        T acc[RP.w];
+#pragma unroll
+        for (int k = 0; k < RP.w; k++)
+          if (RP.r[ph][k] >= 0) acc[k] = y_loc[loc_of(RP.r[ph][k])] + v[RP.r[ph][k]];
+#pragma unroll
+        for (int k = 0; k < RP.w; k++)
+          if (RP.r[ph][k] >= 0) y_loc[loc_of(RP.r[ph][k])] = acc[k];
+      }
+      __syncthreads();
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < NPE; r++) {
+      if (active) y_loc[loc_of(r)] += v[r];
+      __syncthreads();
+    }
   }
 
   // 3. Transposed rows: per node, its terms in sorted order (one segment per node).

@@ -404,4 +404,45 @@ struct TileArgs {
   TileDims dims;
 };
 
+// p = 2: the ranks that a conforming tile's elements add to their points between
+// two barriers.  Let S be the axes on which a rank is a midpoint.  On an axis in S
+// its coordinate is an odd multiple of h / 2, h the element's size, on the
+// others a multiple of h.  Two ranks of two leaves at one position therefore
+// need h_e <= h_f / 2 where S_f has an axis that S_e lacks, and the reverse where
+// S_e has one that S_f lacks, so ranks of different S with equally many
+// axes never meet, whatever the leaves' levels; nor do equal ranks (the leaves
+// would overlap), nor the body rank and any other.  A phase holds one rank of each S of a
+// size (the last one the body rank, too): 14 barriers instead of 27 in 3D, 6
+// instead of 9 in 2D, and up to 4 independent LDS updates between them: 223 us
+// became 219 on the 8.9M-node mesh in FP64.  The traversal's tile kernel, whose
+// missing ranks cost a test each, lost 3 % by it (82,776 elements, one FP32
+// column: 20.8 to 21.6 us) and keeps one rank a phase.
+template <int DIM>
+struct RankPhases {
+  static constexpr int n = DIM == 2 ? 6 : 14, w = DIM + 1;
+  int r[n][w];
+  constexpr RankPhases() : r{} {
+    int ph = 0;
+    for (int size = 0; size < DIM; size++)
+      for (int c = 0; c < 1 << (DIM - size); c++, ph++) {
+        int k = 0;
+        for (int S = 0; S < 1 << DIM; S++) {
+          int bits = 0, rank = 0, p3 = 1, free = c;
+          for (int d = 0; d < DIM; d++, p3 *= 3) {
+            if (S >> d & 1) {
+              bits++;
+              rank += p3;
+            } else {
+              rank += 2 * (free & 1) * p3;
+              free >>= 1;
+            }
+          }
+          if (bits == size) r[ph][k++] = rank;
+        }
+        if (ph == n - 1) r[ph][k++] = (DIM == 2 ? 9 : 27) / 2;
+        for (; k < w; k++) r[ph][k] = -1;
+      }
+  }
+};
+
 }  // namespace dkt
