@@ -100,7 +100,13 @@ __device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int item, cons
   // The weight table's first batch, loaded with the stage loads and stored after them.
   const T w_first = tid < A.nw ? term_w[tid] : T(0);
 
-  // 1. Stage the nodes, then evaluate the hanging points' rows.
+  // 1. Stage the nodes, then evaluate the hanging points' rows (the bounds of
+  // the work-item's first row are loaded here, its terms before the barrier).
+  int r0 = 0, r1 = 0;
+  if (tid < th.nv) {
+    r0 = A.virt_off[th.v0 + tid];
+    r1 = tid + 1 < th.nv ? A.virt_off[th.v0 + tid + 1] : th.nt;
+  }
   const bool active = tid < th.nleaf;
   // The element's local point per rank, two per register; loc_of(r) unpacks
   // one where it is used.  Kept unpacked, the nPe indices would each hold a
@@ -125,33 +131,42 @@ __device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int item, cons
   const int npts = th.nnode + th.nv;
   // Staging in batches of kCB per work-item: every load of a batch is issued
   // before any of its values is used, so a batch costs one memory round trip
-  // after its node ids, not kCB.  The values are loaded before the
-  // Dirichlet flags, and the flags unconditionally (entries past the
-  // tile's nodes read node 0's): a flag tested inside a per-entry branch is
-  // waited for there, one round trip per entry.
-  constexpr int kCB = 4;
+  // after its node ids, not kCB.  The values are loaded before the Dirichlet
+  // flags, and everything unconditionally, entries past the tile's nodes as its
+  // last node's: a load inside a per-entry branch is waited for there.
+  // The kernel is bound by these round trips (73 % of its wave time were
+  // waits), so p = 2 in 3D, with 5 to 8 nodes a work-item, takes 8 at a time, and the
+  // first rows' terms, the segments and the output slots are loaded a phase
+  // early: 218 to 208 us on the 8.9M-node mesh in FP64, 172 to 163 in FP32.
+  // Batches of 4 took 221 us, of 12 (four waves a SIMD instead of five) 232, of 6
+  // 205, but 16.1 for 15.3 at level 6.
+  constexpr int kCB = P == 2 && DIM == 3 ? 8 : 4;
+  const int32_t *nodes = A.tile_nodes + th.node0, *outs = A.tile_out + th.node0;
   for (int j0 = tid; j0 < th.nnode; j0 += kCB * nthr) {
     int g[kCB];
 #pragma unroll
-    for (int b = 0; b < kCB; b++) {
-      const int j = j0 + b * nthr;
-      g[b] = j < th.nnode ? A.tile_nodes[th.node0 + j] : -1;
-    }
+    for (int b = 0; b < kCB; b++) g[b] = nodes[min(j0 + b * nthr, th.nnode - 1)];
     T xv[kCB];
 #pragma unroll
-    for (int b = 0; b < kCB; b++) xv[b] = g[b] >= 0 ? x[(size_t)g[b] * A.ld] : T(0);
+    for (int b = 0; b < kCB; b++) xv[b] = x[(size_t)g[b] * A.ld];
     uint32_t d[kCB];
 #pragma unroll
     for (int b = 0; b < kCB; b++) d[b] = 0u;
     if (A.dir_in)
 #pragma unroll
-      for (int b = 0; b < kCB; b++) d[b] = A.dir_in[g[b] >= 0 ? g[b] : 0];
+      for (int b = 0; b < kCB; b++) d[b] = A.dir_in[g[b]];
 #pragma unroll
     for (int b = 0; b < kCB; b++)
-      if (g[b] >= 0) x_loc[j0 + b * nthr] = d[b] ? T(0) : xv[b];
+      if (j0 + b * nthr < th.nnode) x_loc[j0 + b * nthr] = d[b] ? T(0) : xv[b];
   }
   if (tid < A.nw) wt[tid] = w_first;
   for (int i = tid + nthr; i < A.nw; i += nthr) wt[i] = term_w[i];
+  constexpr int kTB = 4;
+  const uint32_t *tpk = A.term_pk + th.t0;
+  uint32_t e_first[kTB] = {};
+  if (r1 > r0)
+#pragma unroll
+    for (int b = 0; b < kTB; b++) e_first[b] = tpk[min(r0 + b, r1 - 1)];
   __syncthreads();
   // Hanging point values: each row over the staged nodes, terms in row order,
   // read kTB at a time with all loads of a batch issued together.  Entries
@@ -160,15 +175,14 @@ __device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int item, cons
   // cancels to +0), which leaves its bits those of the row's own terms.  A
   // guarded add instead lets the compiler move the load into the guard and
   // wait for it there.
-  constexpr int kTB = 4;
-  const uint32_t *tpk = A.term_pk + th.t0;
   for (int v = tid; v < th.nv; v += nthr) {
-    const int k0 = A.virt_off[th.v0 + v], k1 = v + 1 < th.nv ? A.virt_off[th.v0 + v + 1] : th.nt;
+    const int k0 = v == tid ? r0 : A.virt_off[th.v0 + v];
+    const int k1 = v == tid ? r1 : v + 1 < th.nv ? A.virt_off[th.v0 + v + 1] : th.nt;
     T s = T(0);
     for (int k = k0; k < k1; k += kTB) {
       uint32_t e[kTB];
 #pragma unroll
-      for (int b = 0; b < kTB; b++) e[b] = tpk[min(k + b, k1 - 1)];
+      for (int b = 0; b < kTB; b++) e[b] = k == r0 && v == tid ? e_first[b] : tpk[min(k + b, k1 - 1)];
 #pragma unroll
       for (int b = 0; b < kTB; b++) {
         const T xv = x_loc[e[b] & 0xFFFFu];
@@ -223,6 +237,14 @@ __device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int item, cons
   for (int w = 0; w < NW; w++) asm volatile("" : "+v"(lw[w]));
   __syncthreads();
   for (int j = tid; j < npts; j += nthr) y_loc[j] = T(0);
+  // The first node's segment of step 3 and its terms, loaded while the elements add.
+  const uint32_t *spk = A.term_spk + th.t0;
+  uint32_t sg_first = 0;
+  int m1_first = 0;
+  if (tid < th.ns) {
+    sg_first = A.seg[th.s0 + tid];
+    m1_first = tid + 1 < th.ns ? (int)(A.seg[th.s0 + tid + 1] >> 16) : th.nt;
+  }
   __syncthreads();
   if constexpr (P == 2) {
     constexpr RankPhases<DIM> RP;
@@ -247,12 +269,16 @@ __device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int item, cons
     }
   }
 
+  // Output slots of the first write-out batch, loaded while step 3 runs.
+  int o_first[kCB];
+#pragma unroll
+  for (int b = 0; b < kCB; b++) o_first[b] = outs[min(tid + b * nthr, th.nnode - 1)];
+
   // 3. Transposed rows: per node, its terms in sorted order (one segment per node).
-  const uint32_t *spk = A.term_spk + th.t0;
   for (int g = tid; g < th.ns; g += nthr) {
-    const uint32_t sg = A.seg[th.s0 + g];
+    const uint32_t sg = g == tid ? sg_first : A.seg[th.s0 + g];
     const int j = (int)(sg & 0xFFFFu), m0 = (int)(sg >> 16);
-    const int m1 = g + 1 < th.ns ? (int)(A.seg[th.s0 + g + 1] >> 16) : th.nt;
+    const int m1 = g == tid ? m1_first : g + 1 < th.ns ? (int)(A.seg[th.s0 + g + 1] >> 16) : th.nt;
     T acc = T(0);
     for (int m = m0; m < m1; m += kTB) {
       uint32_t e[kTB];
@@ -272,10 +298,7 @@ __device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int item, cons
   for (int j0 = tid; j0 < th.nnode; j0 += kCB * nthr) {
     int o[kCB];
 #pragma unroll
-    for (int b = 0; b < kCB; b++) {
-      const int j = j0 + b * nthr;
-      o[b] = j < th.nnode ? A.tile_out[th.node0 + j] : INT32_MIN;
-    }
+    for (int b = 0; b < kCB; b++) o[b] = j0 == tid ? o_first[b] : outs[min(j0 + b * nthr, th.nnode - 1)];
     uint32_t d[kCB];
 #pragma unroll
     for (int b = 0; b < kCB; b++) d[b] = 0u;
@@ -285,7 +308,7 @@ __device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int item, cons
 #pragma unroll
     for (int b = 0; b < kCB; b++) {
       const int j = j0 + b * nthr;
-      if (o[b] == INT32_MIN) continue;
+      if (j >= th.nnode) continue;
       if (o[b] >= 0)
         y[(size_t)o[b] * A.ld] = d[b] ? T(0) : y_loc[j];
       else
