@@ -152,7 +152,7 @@ __device__ __forceinline__ T interp_lanes(T a, int lane, int c) {
 // the node-major vectors in L2 (the workgroup may have more work-items than the
 // plan's tile_leaves; they idle in the leaf phases and help in the loops).  A
 // column loop inside the workgroup held the LDS of all columns, which left few
-// workgroups on a CU: eight FP32 columns on 82,776 3D p = 2 elements took 193 us
+// workgroups on a CU: eight FP32 columns on 83,448 3D p = 2 elements took 193 us
 // against 81, eight FP64 ones on the 4D tree of 2M points 23.8 ms against 9.5.
 // ONE: a single column, item = tile; carrying a column index there cost that 4D
 // matvec 1 % in FP64 and 4 % in FP32 (612 to 635 us).
@@ -199,6 +199,13 @@ __device__ __forceinline__ void tile_body(const TileArgs &A, int item, const T *
   const int nthr = blockDim.x;
 
   // 1. Stage.
+  // The loads of a batch are issued together and cost one memory round trip (two
+  // for the nodes: their ids come first), and these trips bound the kernel.  A
+  // p = 2 tile in 3D has about 9 nodes and 5 group slots per work-item, so it
+  // takes 12 and 6 of them at a time: 553k nodes, eight FP32 columns, 82 us with 4 and 2, 77
+  // with 12 and 2, 74 so; 8.9M nodes, one FP64 column, 239, 215, 201.
+  constexpr int kSB = P == 2 && DIM == 3 ? 12 : kNB, kGB = P == 2 && DIM == 3 ? 6 : 2;
+  const int32_t *nodes = A.tile_nodes + th.node0;
   const bool active = tid < th.nleaf;
   uint16_t loc[NPE];
   uint32_t aux = 0;
@@ -212,58 +219,64 @@ __device__ __forceinline__ void tile_body(const TileArgs &A, int item, const T *
   if (tid < TL) ridx_s[tid] = kNone;
   // Output slots of the first write-out batch, loaded with the stage loads so
   // that the write-out does not wait for them.
-  int o_first[kNB];
+  int o_first[kSB];
 #pragma unroll
-  for (int b = 0; b < kNB; b++) {
+  for (int b = 0; b < kSB; b++) {
     const int j = tid + b * nthr;
     o_first[b] = j < th.nnode ? A.tile_out[th.node0 + j] : INT32_MIN;  // INT32_MIN: gathered only
   }
   // Replay block of this lane group's first round, likewise.
   const uint64_t blk_first = (tid / G) < th.nbk ? A.blocks[th.bk0 + tid / G] : 0;
-  // First two batches of the group parent maps and transpose entries, and the
+  // First batches of the group parent maps and transpose entries, and the
   // readers' first batch: loads issued here, stored after the node gathers.
   const int ngp = th.ngrp * NPE;
-  uint16_t gp_first[2];
+  uint16_t gp_first[kGB];
   uint32_t he_first[2];
+  const uint16_t *gpl = A.group_ploc + (size_t)th.grp0 * NPE;
+#pragma unroll
+  for (int b = 0; b < kGB; b++) {
+    const int k = tid + b * nthr;
+    gp_first[b] = k < ngp ? gpl[k] : kNone;
+  }
 #pragma unroll
   for (int b = 0; b < 2; b++) {
     const int k = tid + b * nthr;
-    gp_first[b] = k < ngp ? A.group_ploc[(size_t)th.grp0 * NPE + k] : kNone;
     he_first[b] = k < th.nhe ? A.hentries[th.he0 + k] : 0u;
   }
   const uint16_t rd_first = tid < th.nrd ? A.readers[th.rd0 + tid] : kNone;
-  // Node gathers in batches of kNB per work-item, all loads issued before use:
-  // the first column's values, then the Dirichlet flags, unconditionally
-  // (entries past the tile's nodes read node 0's; a flag tested inside a
-  // per-entry branch is waited for there, one round trip per entry).
-  for (int j0 = tid; j0 < th.nnode; j0 += kNB * nthr) {
-    int g[kNB];
+  // Node gathers in batches of kSB per work-item, all loads issued before use
+  // and unconditionally, entries past the tile's nodes as its last node's (a
+  // load inside a per-entry branch is waited for there; 4D, 2M points, FP32: 611
+  // us with branches, 597 so).
+  for (int j0 = tid; j0 < th.nnode; j0 += kSB * nthr) {
+    int g[kSB];
 #pragma unroll
-    for (int b = 0; b < kNB; b++) {
-      const int j = j0 + b * nthr;
-      g[b] = j < th.nnode ? A.tile_nodes[th.node0 + j] : -1;
-    }
-    T xv[kNB];
+    for (int b = 0; b < kSB; b++) g[b] = nodes[min(j0 + b * nthr, th.nnode - 1)];
+    T xv[kSB];
 #pragma unroll
-    for (int b = 0; b < kNB; b++) xv[b] = g[b] >= 0 ? x[(size_t)g[b] * A.ld] : T(0);
-    uint32_t d[kNB];
+    for (int b = 0; b < kSB; b++) xv[b] = x[(size_t)g[b] * A.ld];
+    uint32_t d[kSB];
 #pragma unroll
-    for (int b = 0; b < kNB; b++) d[b] = 0u;
+    for (int b = 0; b < kSB; b++) d[b] = 0u;
     if (A.dir_in)
 #pragma unroll
-      for (int b = 0; b < kNB; b++) d[b] = A.dir_in[g[b] >= 0 ? g[b] : 0];
+      for (int b = 0; b < kSB; b++) d[b] = A.dir_in[g[b]];
 #pragma unroll
-    for (int b = 0; b < kNB; b++)
-      if (g[b] >= 0) x_loc[j0 + b * nthr] = d[b] ? T(0) : xv[b];
+    for (int b = 0; b < kSB; b++)
+      if (j0 + b * nthr < th.nnode) x_loc[j0 + b * nthr] = d[b] ? T(0) : xv[b];
+  }
+#pragma unroll
+  for (int b = 0; b < kGB; b++) {
+    const int k = tid + b * nthr;
+    if (k < ngp) gploc[k] = gp_first[b];
   }
 #pragma unroll
   for (int b = 0; b < 2; b++) {
     const int k = tid + b * nthr;
-    if (k < ngp) gploc[k] = gp_first[b];
     if (k < th.nhe) hent[k] = he_first[b];
   }
   if (tid < th.nrd) rdl_s[tid] = rd_first;
-  for (int k = tid + 2 * nthr; k < ngp; k += nthr) gploc[k] = A.group_ploc[(size_t)th.grp0 * NPE + k];
+  for (int k = tid + kGB * nthr; k < ngp; k += nthr) gploc[k] = gpl[k];
   for (int k = tid + 2 * nthr; k < th.nhe; k += nthr) hent[k] = A.hentries[th.he0 + k];
   for (int k = tid + nthr; k < th.nrd; k += nthr) rdl_s[k] = A.readers[th.rd0 + k];
   const bool hang = active && aux_hang(aux);
@@ -457,21 +470,21 @@ __device__ __forceinline__ void tile_body(const TileArgs &A, int item, const T *
   }
   __syncthreads();
   // 7. Write out: owned nodes to y, shared nodes to their partial slot.
-  for (int j0 = tid; j0 < th.nnode; j0 += kNB * nthr) {
-    int o[kNB];
+  for (int j0 = tid; j0 < th.nnode; j0 += kSB * nthr) {
+    int o[kSB];
 #pragma unroll
-    for (int b = 0; b < kNB; b++) {
+    for (int b = 0; b < kSB; b++) {
       const int j = j0 + b * nthr;
       o[b] = j0 == tid ? o_first[b] : (j < th.nnode ? A.tile_out[th.node0 + j] : INT32_MIN);
     }
-    uint32_t d[kNB];  // Dirichlet flags, loaded unconditionally as in the stage
+    uint32_t d[kSB];  // Dirichlet flags, loaded unconditionally as in the stage
 #pragma unroll
-    for (int b = 0; b < kNB; b++) d[b] = 0u;
+    for (int b = 0; b < kSB; b++) d[b] = 0u;
     if (A.dir_out)
 #pragma unroll
-      for (int b = 0; b < kNB; b++) d[b] = A.dir_out[o[b] >= 0 ? o[b] : 0];
+      for (int b = 0; b < kSB; b++) d[b] = A.dir_out[o[b] >= 0 ? o[b] : 0];
 #pragma unroll
-    for (int b = 0; b < kNB; b++) {
+    for (int b = 0; b < kSB; b++) {
       const int j = j0 + b * nthr;
       if (o[b] == INT32_MIN) continue;
       const T acc = y_loc[j];
