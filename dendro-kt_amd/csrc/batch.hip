@@ -32,6 +32,26 @@ struct GroupBase {
   virtual void launch(hipStream_t st) = 0;
 };
 
+// launch(first, count) over the items of a group, in as many launches as their
+// work-items need.
+template <typename F>
+void launch_items(int nitems, int threads, const F &launch) {
+  const int most = (int)std::min<size_t>(INT32_MAX, max_groups_of(std::max(1, threads)));
+  for (int first = 0; first < nitems;) {
+    const int count = std::min(most, nitems - first);
+    launch(first, count);
+    HIP_OK(hipGetLastError());
+    first += count;
+  }
+}
+
+// First items of a group's records: adds a record's items to their sum, which
+// must stay a 32-bit index.
+inline void push_items(std::vector<int> &start, size_t items) {
+  if (start.back() + items > (size_t)INT32_MAX) throw std::invalid_argument("too many tiles and columns in a batch");
+  start.push_back(start.back() + (int)items);
+}
+
 // Device copies of a group's tables: in the caller's arena when there is one,
 // else in buffers the group owns.
 struct GroupMem {
@@ -149,7 +169,7 @@ struct Group : GroupBase, FixSource<T> {
         threads = std::max(threads, pl->tile_leaves);
         poff.push_back(ptot);
         ptot += pl->npartial * (size_t)chunk;
-        ts.push_back(ts.back() + (int)pl->ntiles * std::min(chunk, nrhs - c * chunk));
+        push_items(ts, pl->ntiles * (size_t)std::min(chunk, nrhs - c * chunk));
       }
     partial = mem.alloc<T>(std::max<size_t>(1, ptot));
     one = chunk == 1;
@@ -200,10 +220,10 @@ struct Group : GroupBase, FixSource<T> {
   }
 
   void launch(hipStream_t st) override {
-    if (ntiles)
-      hipLaunchKernelGGL((one ? tile_kernel_batch<T, DIM, P, true> : tile_kernel_batch<T, DIM, P, false>),
-                         dim3(ntiles), dim3(threads), lds, st, table, tile_start, nrec);
-    HIP_OK(hipGetLastError());
+    auto kernel = one ? tile_kernel_batch<T, DIM, P, true> : tile_kernel_batch<T, DIM, P, false>;
+    launch_items(ntiles, threads, [&](int first, int count) {
+      hipLaunchKernelGGL(kernel, dim3(count), dim3(threads), lds, st, table, tile_start, nrec, first);
+    });
   }
 };
 
@@ -218,8 +238,9 @@ struct PointBatchPlan {
 // All tiles and columns of a batch of point plans of one dim in one launch.
 template <typename T, int DIM, bool CAP>
 __global__ void __launch_bounds__(kTileThreads) point_kernel_batch(const PointBatchPlan<T> *__restrict__ plans,
-                                                                   const int *__restrict__ item_start, int nplans) {
-  const int t = xcd_tile(blockIdx.x, gridDim.x);
+                                                                   const int *__restrict__ item_start, int nplans,
+                                                                   int first) {
+  const int t = first + xcd_tile(blockIdx.x, gridDim.x);
   const int k = find_range(item_start, nplans, t);
   const PointBatchPlan<T> bp = plans[k];  // a copy: its fields live in scalar registers
   if (bp.A.cancel && *bp.A.cancel) return;
@@ -260,7 +281,7 @@ struct PointGroup : GroupBase, FixSource<T> {
                                        (const T *)xs[k] + coff, (T *)ys[k] + coff, nullptr});
         poff.push_back(ptot);
         ptot += pl->npartial * (size_t)nq;
-        is.push_back(is.back() + (int)pl->ntiles * nq);
+        push_items(is, pl->ntiles * (size_t)nq);
       }
     }
     partial = mem.alloc<T>(std::max<size_t>(1, ptot));
@@ -277,9 +298,10 @@ struct PointGroup : GroupBase, FixSource<T> {
   }
 
   void launch(hipStream_t st) override {
-    if (nitems)
-      hipLaunchKernelGGL((point_kernel_batch<T, DIM, CAP>), dim3(nitems), dim3(threads), lds, st, table, item_start, nrec);
-    HIP_OK(hipGetLastError());
+    launch_items(nitems, threads, [&](int first, int count) {
+      hipLaunchKernelGGL((point_kernel_batch<T, DIM, CAP>), dim3(count), dim3(threads), lds, st, table, item_start, nrec,
+                         first);
+    });
   }
 };
 
@@ -295,8 +317,8 @@ struct ConfBatchPlan {
 template <typename T, int DIM, int P, bool CAP>
 __global__ void __launch_bounds__(kTileThreads) conf_tile_kernel_batch(const ConfBatchPlan<T> *__restrict__ plans,
                                                                        const int *__restrict__ tile_start,
-                                                                       int nplans) {
-  const int t = xcd_tile(blockIdx.x, gridDim.x);
+                                                                       int nplans, int first) {
+  const int t = first + xcd_tile(blockIdx.x, gridDim.x);
   const int k = find_range(tile_start, nplans, t);
   const ConfBatchPlan<T> bp = plans[k];  // a copy: its fields live in scalar registers
   if (bp.A.cancel && *bp.A.cancel) return;
@@ -335,7 +357,7 @@ struct ConfGroup : GroupBase, FixSource<T> {
         threads = std::max(threads, pl->tile_leaves);
         poff.push_back(ptot);
         ptot += pl->npartial * (size_t)chunk;
-        ts.push_back(ts.back() + (int)pl->ntiles * std::min(chunk, nrhs - c * chunk));
+        push_items(ts, pl->ntiles * (size_t)std::min(chunk, nrhs - c * chunk));
       }
     partial = mem.alloc<T>(std::max<size_t>(1, ptot));
     std::vector<ConfBatchPlan<T>> hp(pls.size() * nchunks);
@@ -385,10 +407,10 @@ struct ConfGroup : GroupBase, FixSource<T> {
   }
 
   void launch(hipStream_t st) override {
-    if (ntiles)
-      hipLaunchKernelGGL((conf_tile_kernel_batch<T, DIM, P, CAP>), dim3(ntiles), dim3(threads), lds, st, table,
-                         tile_start, nrec);
-    HIP_OK(hipGetLastError());
+    launch_items(ntiles, threads, [&](int first, int count) {
+      hipLaunchKernelGGL((conf_tile_kernel_batch<T, DIM, P, CAP>), dim3(count), dim3(threads), lds, st, table,
+                         tile_start, nrec, first);
+    });
   }
 };
 

@@ -1312,7 +1312,7 @@ template <typename T>
 int launch_columns(const dkt_plan *pl, int nrhs, const ExtScratch *ext) {
   int chunk = std::min(nrhs, kCols);
   while (ext && chunk > 1 && pl->npartial * (size_t)chunk * sizeof(T) > ext->bytes) chunk--;
-  if (pl->ntiles * (size_t)chunk > (size_t)INT32_MAX) throw std::invalid_argument("too many tiles and columns");
+  while (chunk > 1 && pl->ntiles * (size_t)chunk > max_groups_of(pl->tile_leaves)) chunk--;
   return chunk;
 }
 

@@ -404,6 +404,10 @@ struct TileArgs {
   TileDims dims;
 };
 
+// Workgroups of `threads` work-items that one launch may have (a launch counts its
+// work-items in 32 bits).
+inline size_t max_groups_of(int threads) { return (size_t)UINT32_MAX / (size_t)threads; }
+
 // p = 2: the ranks that a conforming tile's elements add to their points between
 // two barriers.  Let S be the axes on which a rank is a midpoint.  On an axis in S
 // its coordinate is an odd multiple of h / 2, h the element's size, on the

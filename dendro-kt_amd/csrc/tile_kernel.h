@@ -539,11 +539,11 @@ __device__ __forceinline__ int find_range(const int *__restrict__ starts, int n,
 }
 
 // All tiles and columns of a batch of same-(dim, p) plans in one launch: batch
-// item t = xcd_tile(b) of workgroup b is item t - tile_start[k] of plan k.
+// item t = first + xcd_tile(b) of workgroup b is item t - tile_start[k] of plan k.
 template <typename T, int DIM, int P, bool ONE>
 __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(tile_waves<T, DIM, P>())))
-tile_kernel_batch(const BatchPlan<T> *__restrict__ plans, const int *__restrict__ tile_start, int nplans) {
-  const int t = xcd_tile(blockIdx.x, gridDim.x);
+tile_kernel_batch(const BatchPlan<T> *__restrict__ plans, const int *__restrict__ tile_start, int nplans, int first) {
+  const int t = first + xcd_tile(blockIdx.x, gridDim.x);
   const int k = find_range(tile_start, nplans, t);
   const BatchPlan<T> bp = plans[k];  // a copy: its fields live in scalar registers
   if (bp.A.cancel && *bp.A.cancel) return;
