@@ -53,8 +53,9 @@ extern "C" {
  * per-leaf/per-node kernels with DKT_PLAN_SIMPLE. */
 #define DKT_PLAN_CONFORMING 4
 /* Leaves per tile of the tiled path: flags |= log2(leaves) << DKT_PLAN_TILE_SHIFT
- * with leaves in {64, 128, 256}; 0 = 128, halved while the LDS footprint does
- * not fit.  Tiles also end early at 32 stale-buffer readers. */
+ * with leaves in {64, 128, 256}; 0 = 256 for p = 1 in 2D and 3D, else 128,
+ * halved while the LDS footprint does not fit.  Tiles also end early at 32
+ * stale-buffer readers. */
 #define DKT_PLAN_TILE_SHIFT 8
 
 typedef struct dkt_octs dkt_octs; /* host list of cells/points */
@@ -320,13 +321,12 @@ typedef struct dkt_batch dkt_batch;
  * and the cause is not found). */
 #define DKT_BATCH_PERSISTENT 2
 /* Columns per tile record for nrhs > 1: flags |= (log2(columns) + 1) <<
- * DKT_BATCH_COLUMNS_SHIFT with columns in {1, 2, 4, ..., 64}; 0 = as many
- * as the tiles' LDS allows.  The columns are cut into chunks of that many,
- * each chunk a record of the same launch (one tile launch and one fix-up
- * launch per (dim, p) group).  One column per record runs the single-column
- * tile kernels (fewer registers, more waves per SIMD) over the same
- * [N][nrhs] vectors; the autotuner chooses it per (dim, p).  Each column's
- * result is bitwise the same either way. */
+ * DKT_BATCH_COLUMNS_SHIFT with columns in {1, 2, 4, ..., 64}; 0 = all of
+ * them.  The columns are cut into chunks of that many, each chunk a record of
+ * the same launch (one tile launch and one fix-up launch per (dim, p) group);
+ * every column of a chunk is a workgroup of its own per tile.  The autotuner
+ * chooses it per (dim, p).  Each column's result is bitwise the same either
+ * way. */
 #define DKT_BATCH_COLUMNS_SHIFT 8
 /* x[k], y[k] column-major, [nrhs][N_k] (column q at q * N_k), instead of
  * [N_k][nrhs]: every (column, plan) pair is a single-column record (the
