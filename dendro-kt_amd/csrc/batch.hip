@@ -30,6 +30,7 @@ namespace {
 struct GroupBase {
   virtual ~GroupBase() = default;
   virtual void launch(hipStream_t st) = 0;
+  double ranks = 0;  // leaf ranks of the group's items: its work, to order launches by
 };
 
 // launch(first, count) over the items of a group, in as many launches as their
@@ -170,6 +171,7 @@ struct Group : GroupBase, FixSource<T> {
         poff.push_back(ptot);
         ptot += pl->npartial * (size_t)chunk;
         push_items(ts, pl->ntiles * (size_t)std::min(chunk, nrhs - c * chunk));
+        ranks += (double)pl->L * NPE * std::min(chunk, nrhs - c * chunk);
       }
     partial = mem.alloc<T>(std::max<size_t>(1, ptot));
     one = chunk == 1;
@@ -282,6 +284,7 @@ struct PointGroup : GroupBase, FixSource<T> {
         poff.push_back(ptot);
         ptot += pl->npartial * (size_t)nq;
         push_items(is, pl->ntiles * (size_t)nq);
+        ranks += (double)pl->L * pl->npe * nq;
       }
     }
     partial = mem.alloc<T>(std::max<size_t>(1, ptot));
@@ -358,6 +361,7 @@ struct ConfGroup : GroupBase, FixSource<T> {
         poff.push_back(ptot);
         ptot += pl->npartial * (size_t)chunk;
         push_items(ts, pl->ntiles * (size_t)std::min(chunk, nrhs - c * chunk));
+        ranks += (double)pl->L * NPE * std::min(chunk, nrhs - c * chunk);
       }
     partial = mem.alloc<T>(std::max<size_t>(1, ptot));
     std::vector<ConfBatchPlan<T>> hp(pls.size() * nchunks);
@@ -502,7 +506,7 @@ std::unique_ptr<MatvecLauncher> dkt::batch_matvec(int dtype, const std::vector<d
 }
 
 struct dkt_batch {
-  std::vector<std::unique_ptr<GroupBase>> groups;
+  std::vector<std::unique_ptr<GroupBase>> groups;  // the most work first
   std::unique_ptr<FixLaunchBase> fixes;  // the shared nodes of every group, after their tiles
   void launch(hipStream_t st) {
     for (auto &g : groups) g->launch(st);
@@ -512,13 +516,24 @@ struct dkt_batch {
   // partial slots and outputs are disjoint), so each goes on a branch of its
   // own, forked from and joined back to the caller's stream before the
   // fix-up; the replayed graph may then run them side by side.  The branch
-  // streams have the default priority.
+  // streams have the default priority.  The group with the most work is recorded
+  // first: in a replay a branch starts 9 to 20 us behind the one recorded before
+  // it, which a long launch hides and a short one does not (24 trees of up to 35k
+  // elements, p = 1 and 2 in turn, one FP32 column: 34.0 us, with the p = 1 group
+  // first 46.2, with both on one stream 44.6; 8 FP64 columns on 18 trees of up to
+  // 11k: 79.4, 88.3 and 90.5).
+  // Large FP32 batches stay on one stream: side by side the launches slow each
+  // other down by more than the overlap of their ends gains (182M leaf ranks: 535 us
+  // against 522, 122M 374 and 369, 102M 318 and 317, but 68M 202 and 208; in FP64 182M
+  // 976 and 994).
+  static constexpr double kBranchRanks32 = 1e8;
+  bool branches = false;
   std::vector<hipStream_t> branch;
   std::vector<hipEvent_t> done;
   hipEvent_t fork = nullptr;
   // Streams and events of the branches, made before the capture starts.
   void prepare_branches() {
-    if (fork || groups.size() < 2) return;
+    if (fork || !branches) return;
     HIP_OK(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
     for (size_t g = 1; g < groups.size(); g++) {
       hipStream_t s2 = nullptr;
@@ -530,18 +545,18 @@ struct dkt_batch {
     }
   }
   void capture(hipStream_t st) {
-    if (groups.size() < 2 || !fork) {
+    if (!branches || done.size() + 1 != groups.size()) {
       launch(st);
       return;
     }
     HIP_OK(hipEventRecord(fork, st));
-    for (size_t g = 1; g < groups.size(); g++) {
-      HIP_OK(hipStreamWaitEvent(branch[g - 1], fork, 0));
-      groups[g]->launch(branch[g - 1]);
-      HIP_OK(hipEventRecord(done[g - 1], branch[g - 1]));
+    for (size_t g = 0; g < done.size(); g++) {
+      HIP_OK(hipStreamWaitEvent(branch[g], fork, 0));
+      groups[g]->launch(branch[g]);
+      HIP_OK(hipEventRecord(done[g], branch[g]));
     }
-    groups[0]->launch(st);
-    for (size_t g = 1; g < groups.size(); g++) HIP_OK(hipStreamWaitEvent(st, done[g - 1], 0));
+    groups.back()->launch(st);
+    for (hipEvent_t e : done) HIP_OK(hipStreamWaitEvent(st, e, 0));
     if (fixes) fixes->launch(st);
   }
   bool use_graph = false;
@@ -591,6 +606,11 @@ extern "C" int dkt_batch_create(dkt_plan *const *plans, int nplans, int dtype, i
                          : make_group<float>(conf, dim, p, pls, xs, ys, nrhs, masked, {}, nullptr, max_cols, cm);
       b->groups.emplace_back(g);
     }
+    std::stable_sort(b->groups.begin(), b->groups.end(),
+                     [](const auto &a, const auto &c) { return a->ranks > c->ranks; });
+    double ranks = 0;
+    for (const auto &g : b->groups) ranks += g->ranks;
+    b->branches = b->groups.size() > 1 && (dtype == 0 || ranks <= dkt_batch::kBranchRanks32);
     b->fixes = dtype == 0 ? fix_all<double>(b->groups, nullptr) : fix_all<float>(b->groups, nullptr);
     b->use_graph = (flags & DKT_BATCH_GRAPH) != 0;
     *out = b.release();
