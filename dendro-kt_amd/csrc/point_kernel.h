@@ -96,20 +96,25 @@ __device__ __forceinline__ void replay(const PtTile &th, T *P, const unsigned ch
   const int tid = threadIdx.x, nthr = blockDim.x;
   for (int i = tid; i < th.ngrp * NPE; i += nthr) pval[i] = P[gp[i] != kNone ? gp[i] : 0];  // absent: not used
   // Buffer state at the tile start: slot s sums its terms (a header of slot
-  // offsets, then the terms by slot), dealt to the R lanes of the slot.
-  {
-    const int R = nthr / NPE, slot = tid / R, sub = tid % R;  // R = 4 .. 64 lanes, a power of two
+  // offsets, then the terms by slot), dealt to the R lanes of the slot.  R is
+  // the plan's, not the workgroup's, so that the order of the sum does not
+  // depend on the launch: a batch's workgroups have the work-items of its
+  // largest tiles, NPE * R or more (those past them do the last slot again).
+  if (th.ncr > 0) {
+    const int lg = th.carry_log(), R = 1 << lg, slot = min(tid >> lg, NPE - 1), sub = tid & (R - 1);  // R = 4 .. 64
     const double *cw = reinterpret_cast<const double *>(block + th.carry_w_at());
     const uint32_t *ck = reinterpret_cast<const uint32_t *>(block + th.carry_key_at());
-    const int lo = th.ncr > 0 ? (int)ck[slot] : 0, hi = th.ncr > 0 ? (int)ck[slot + 1] : 0;
+    const int lo = (int)ck[slot], hi = (int)ck[slot + 1];
     T acc = T(0);
     for (int c = lo + sub; c < hi; c += R) acc += (T)cw[c] * P[ck[c] & 0xFFFFu];
     for (int d = R >> 1; d; d >>= 1) acc += __shfl_xor(acc, d, 64);
     if (!sub) cst[slot] = acc;
+  } else if (tid < NPE) {
+    cst[tid] = T(0);
   }
   __syncthreads();
   const int lane = tid % G, ngroups = nthr / G;
-  for (int bi = tid / G; bi < th.nbk; bi += ngroups) {
+  for (int bi = tid / G; bi < th.nbk(); bi += ngroups) {
     const uint64_t blk = blocks[bi];
     const int S = (int)(blk & 0xFFFFu), E = (int)((blk >> 16) & 0xFFFFu);
     const uint32_t r0 = ((uint32_t)(blk >> 32) & 0xFFFFu) + 1, nr = (uint32_t)(blk >> 48);  // the block's readers (+ 1)
@@ -229,7 +234,7 @@ __device__ __forceinline__ void point_body(const PtArgs &A, int item, const T *_
   const uint32_t rw_odd = tid < nlist ? rows[nrow + tid] : 0u;
   if (nlist) {
     for (int i = tid; i < th.nodd; i += nthr) row(nrow + i);
-    if (th.nbk) replay<T, DIM>(th, P, block, reinterpret_cast<T *>(block + (size_t)A.max_units * 16));
+    if (th.nbk()) replay<T, DIM>(th, P, block, reinterpret_cast<T *>(block + (size_t)A.max_units * 16));
     __syncthreads();
   }
   block_copy(block, A.blocks + (size_t)th.b0 * 4, th.nb);

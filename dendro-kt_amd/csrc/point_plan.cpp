@@ -301,7 +301,8 @@ void for_tiles(size_t ntiles, F &&work) {
 
 // Partial slots of the nodes that several tiles write (consecutive per node,
 // in tile order) and the tiles' blocks.
-void concatenate(PointHost &o, std::vector<TileOut> &outs, size_t N, int npe) {
+void concatenate(PointHost &o, std::vector<TileOut> &outs, size_t N, int T, int npe) {
+  const int carry_log = __builtin_ctz((unsigned)(T / npe));
   std::vector<int32_t> ntarget(N, 0);
   for (const TileOut &to : outs)
     for (size_t j = 0; j < to.nodes.size(); j++)
@@ -329,7 +330,7 @@ void concatenate(PointHost &o, std::vector<TileOut> &outs, size_t N, int npe) {
     h.nstep = (int32_t)to.step.size();
     h.nquad = (int32_t)to.quads.size();
     h.nrd = (int32_t)to.rdr.size();
-    h.nbk = (int32_t)to.blk.size();
+    h.rep = (int32_t)to.blk.size() | carry_log << 16;
     h.ncr = (int32_t)to.ckey.size();
     h.ngrp = (int32_t)(to.gploc.size() / npe);
     h.nch = (int32_t)to.chain.size();
@@ -745,7 +746,7 @@ PointHost build_points_reference(const MeshParams &mp, const Traversal &tr, size
       to.rdr.push_back((uint64_t)sc.rn.point[q.point] | (uint64_t)q.mask << 32);
   };
   for_tiles<Scratch>(ntiles, build_tile);
-  concatenate(o, outs, N, npe);
+  concatenate(o, outs, N, T, npe);
   return o;
 }
 
@@ -911,7 +912,7 @@ bool build_points_conforming(const MeshParams &mp, const Traversal &tr, const st
   } catch (const Misfit &) {
     return false;
   }
-  concatenate(o, outs, N, npe);
+  concatenate(o, outs, N, T, npe);
   out = std::move(o);
   return true;
 }

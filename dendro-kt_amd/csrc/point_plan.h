@@ -40,14 +40,18 @@ struct PtTile {
   int32_t ncor;          // correction slots, after the points; then the zero slot
   int32_t nstep, nquad;  // step words (an even number), quads
   int32_t nqs;           // groups of four steps onto the nodes
-  int32_t nrd, nbk, ncr, ngrp, nch;  // replay: readers, blocks, carry terms, sibling groups, chain words
+  int32_t nrd, rep, ncr, ngrp, nch;  // replay: readers, blocks and carry_log() << 16, carry terms, sibling groups, chain words
+  constexpr int32_t nbk() const { return rep & 0xFFFF; }
+  // log2 of the lanes that sum one slot of the buffer state at the tile start: those
+  // of a workgroup of the plan's leaves per tile, whatever the launch has.
+  constexpr int32_t carry_log() const { return rep >> 16; }
   constexpr int32_t past(int k) const { return (int32_t)(lv[k] & 0xFFFFu); }
   constexpr int32_t npts() const { return nrow + nodd + nrdp; }
   // Byte offsets in block A and B.
   constexpr int32_t rows_at() const { return 8 * nnode; }
   constexpr int32_t readers_at() const { return (8 * nnode + 4 * (npts() - nnode) + 7) & ~7; }
   constexpr int32_t blocks_at() const { return readers_at() + 8 * nrd; }
-  constexpr int32_t carry_w_at() const { return blocks_at() + 8 * nbk; }
+  constexpr int32_t carry_w_at() const { return blocks_at() + 8 * nbk(); }
   constexpr int32_t carry_key_at() const { return carry_w_at() + 8 * ncr; }
   constexpr int32_t chain_at() const { return carry_key_at() + 4 * ncr; }
   constexpr int32_t gploc_at() const { return chain_at() + 4 * nch; }
