@@ -464,6 +464,7 @@ PointHost build_points_reference(const MeshParams &mp, const Traversal &tr, size
         bounds.push_back(e);
         nrd = 0;
         ngrp = 0;
+        new_group = hang;  // of the new tile, also where the last one ended inside the group
       }
       nrd += reader ? 1 : 0;
       ngrp += new_group ? 1 : 0;
