@@ -927,13 +927,15 @@ size_t size_points(dkt_plan *pl, const PointHost &o) {
   return pl->lds_bytes = point_lds<double>(pl);
 }
 
-// Leaves per tile: the requested size, else kPointTile, halved until the LDS
-// footprint (FP64) fits.
+// Leaves per tile: the requested size, else kPointTile, halved until the tiles fit
+// the layout and their LDS footprint (FP64) the limit.
 void build_points(dkt_plan *pl, const MeshParams &mp, const Traversal &tr, int requested) {
   int T = requested ? requested : kPointTile;
   while (true) {
-    PointHost o = build_points_reference(mp, tr, pl->N, T, std::max(1, T / pl->npe));
-    if (size_points(pl, o) <= kLdsLimit) return upload_points(pl, o, T);
+    PointHost o;
+    if (build_points_reference(mp, tr, pl->N, T, std::max(1, T / pl->npe), o) == PtFit::yes &&
+        size_points(pl, o) <= kLdsLimit)
+      return upload_points(pl, o, T);
     if (requested || T <= 64) throw std::runtime_error("tile does not fit in LDS");
     T /= 2;
   }
@@ -946,8 +948,9 @@ void build_points(dkt_plan *pl, const MeshParams &mp, const Traversal &tr, int r
 bool build_conf_points(dkt_plan *pl, const MeshParams &mp, const Traversal &tr, const NodeSet &ns, int T) {
   for (; T >= 64; T /= 2) {
     PointHost o;
-    if (!build_points_conforming(mp, tr, ns.nodes, T, kMaxConfTerms, o)) continue;
-    if (size_points(pl, o) > kLdsLimit) continue;
+    const PtFit fit = build_points_conforming(mp, tr, ns.nodes, T, kMaxConfTerms, o);
+    if (fit == PtFit::none) break;
+    if (fit != PtFit::yes || size_points(pl, o) > kLdsLimit) continue;
     upload_points(pl, o, T);
     return true;
   }

@@ -35,6 +35,12 @@ namespace {
 constexpr uint16_t kAbsent = 0xFFFF;
 constexpr int kMaxTileReaders = 32;  // stale-buffer readers per tile (6 bits of a chain word)
 
+// A tile that does not fit the layout.  smaller: one of fewer leaves may.
+struct Misfit : std::runtime_error {
+  bool smaller;
+  explicit Misfit(const char *what, bool smaller = true) : std::runtime_error(what), smaller(smaller) {}
+};
+
 // Tile-local numbering of global ids (first touch): open addressing, cleared
 // in time proportional to its use.
 struct LocalIds {
@@ -51,7 +57,7 @@ struct LocalIds {
     while (key[h] != -1 && key[h] != n) h = (h + 1) & mask;
     *fresh = key[h] == -1;
     if (*fresh) {
-      if (used.size() * 2 >= key.size()) throw std::runtime_error("tile has too many nodes");
+      if (used.size() * 2 >= key.size()) throw Misfit("tile has too many nodes");
       key[h] = n;
       val[h] = (int32_t)used.size();
       used.push_back(h);
@@ -99,7 +105,7 @@ struct PointSet {
         return k;
       k = (k + 1) & mask;
     }
-    if (used.size() * 2 >= table.size()) throw std::runtime_error("tile has too many points");
+    if (used.size() * 2 >= table.size()) throw Misfit("tile has too many points");
     used.push_back(k);
     return k;
   }
@@ -131,11 +137,6 @@ struct Renumber {
   uint16_t operator()(int32_t ref) const { return ref >= 0 ? node[ref] : point[-1 - ref]; }
 };
 
-// A tile that does not fit the layout.
-struct Misfit : std::runtime_error {
-  using std::runtime_error::runtime_error;
-};
-
 // Orders a tile's nodes and points and writes its rows and sums.  In: nodes by
 // first touch, the points, corr: the node of each correction slot.
 void finish_tile(TileOut &to, PointSet &ps, const std::vector<uint16_t> &corr, Renumber &rn) {
@@ -151,7 +152,7 @@ void finish_tile(TileOut &to, PointSet &ps, const std::vector<uint16_t> &corr, R
     lev[i] = (uint8_t)(1 + std::max(la, lb));
     nlev = std::max(nlev, (int)lev[i]);
   }
-  if (nlev > kPtLevels) throw Misfit("tile has too many row levels");
+  if (nlev > kPtLevels) throw Misfit("tile has too many row levels", false);  // a leaf's chain, whatever the tile
   for (size_t i = np; i-- > 0;) {  // the ends of a live row are live
     const Point &p = ps.pts[i];
     if (p.kind == kRow && p.live)
@@ -253,7 +254,7 @@ void finish_tile(TileOut &to, PointSet &ps, const std::vector<uint16_t> &corr, R
         }
         words.push_back(w);
       }
-      if (first > 0xFFFF) throw std::runtime_error("tile has too many transposed terms");
+      if (first > 0xFFFF) throw Misfit("tile has too many transposed terms");
       to.step.push_back((uint32_t)first | (uint32_t)(t - t0) << 16);
     }
     for (; steps % per; steps++) to.step.push_back(0);  // groups of four quads, two pairs
@@ -397,13 +398,26 @@ void concatenate(PointHost &o, std::vector<TileOut> &outs, size_t N, int T, int 
   });
 }
 
+// Builds every tile (build_tile fills outs) and, where all fit, the plan's arrays.
+template <typename Scratch, typename F>
+PtFit finish(PointHost &o, std::vector<TileOut> &outs, size_t N, int T, int npe, F &&build_tile, PointHost &out) {
+  try {
+    for_tiles<Scratch>(outs.size(), build_tile);
+  } catch (const Misfit &m) {
+    return m.smaller ? PtFit::smaller : PtFit::none;
+  }
+  concatenate(o, outs, N, T, npe);
+  out = std::move(o);
+  return PtFit::yes;
+}
+
 }  // namespace
 
 size_t PointHost::bytes() const {
   return tiles.size() * sizeof(PtTile) + snode.size() * 8 + lloc.size() * 2 + (laux.size() + blocks.size()) * 4;
 }
 
-PointHost build_points_reference(const MeshParams &mp, const Traversal &tr, size_t N, int T, int n_groups) {
+PtFit build_points_reference(const MeshParams &mp, const Traversal &tr, size_t N, int T, int n_groups, PointHost &out) {
   const int dim = mp.dim, npe = tr.nPe;
   const size_t L = tr.leaves.size();
   StaleBuffer sb(mp, tr);
@@ -710,7 +724,7 @@ PointHost build_points_reference(const MeshParams &mp, const Traversal &tr, size
           cpar = par;
           const int32_t *ps = &tr.pslot[(size_t)tr.hang_of[e] * npe];
           for (int s = 0; s < npe; s++) to.gploc.push_back(ps[s] >= 0 ? node(ps[s], false) : kAbsent);
-          if (g > 63) throw std::runtime_error("tile has too many sibling groups");
+          if (g > 63) throw Misfit("tile has too many sibling groups");
         }
         uint32_t missing, absent;
         masks(e, &missing, &absent);
@@ -746,12 +760,10 @@ PointHost build_points_reference(const MeshParams &mp, const Traversal &tr, size
     for (const Rd &q : rd)
       to.rdr.push_back((uint64_t)sc.rn.point[q.point] | (uint64_t)q.mask << 32);
   };
-  for_tiles<Scratch>(ntiles, build_tile);
-  concatenate(o, outs, N, T, npe);
-  return o;
+  return finish<Scratch>(o, outs, N, T, npe, build_tile, out);
 }
 
-bool build_points_conforming(const MeshParams &mp, const Traversal &tr, const std::vector<Oct> &nodes, int T,
+PtFit build_points_conforming(const MeshParams &mp, const Traversal &tr, const std::vector<Oct> &nodes, int T,
                              int max_terms, PointHost &out) {
   const int dim = mp.dim, npe = tr.nPe;
   const size_t E = tr.leaves.size(), N = nodes.size();
@@ -908,14 +920,7 @@ bool build_points_conforming(const MeshParams &mp, const Traversal &tr, const st
     if (2 * (to.h.nrow - to.h.nnode) > max_terms) throw Misfit("tile has too many row ends");
     for (size_t i = 0; i < (l1 - l0) * npe; i++) o.lloc[l0 * npe + i] = sc.rn(sc.ref[i]);
   };
-  try {
-    for_tiles<Scratch>(ntiles, build_tile);
-  } catch (const Misfit &) {
-    return false;
-  }
-  concatenate(o, outs, N, T, npe);
-  out = std::move(o);
-  return true;
+  return finish<Scratch>(o, outs, N, T, npe, build_tile, out);
 }
 
 }  // namespace dkt

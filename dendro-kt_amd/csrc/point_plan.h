@@ -90,16 +90,19 @@ struct PointHost {
   size_t bytes() const;
 };
 
+// Whether a mesh's tiles fit the layout (the limits above): yes, perhaps with
+// fewer leaves per tile, or with none.
+enum class PtFit { yes, smaller, none };
+
 // Reference semantics over the flattened traversal, tiles of at most T leaves;
 // n_groups: replay blocks per tile.
-PointHost build_points_reference(const MeshParams &mp, const Traversal &tr, size_t N, int T, int n_groups);
+PtFit build_points_reference(const MeshParams &mp, const Traversal &tr, size_t N, int T, int n_groups, PointHost &out);
 
 // Conforming operator (sum_e C_e^T K_e C_e, build_conforming): a rank that is no
 // node takes its parent cell's interpolant, whose corners do the same one level
-// up, so every hanging point is a row.  Tiles of T elements.  Returns false where
-// a tile does not fit the layout (more row levels than kPtLevels, or more than
-// max_terms ends of rows).
-bool build_points_conforming(const MeshParams &mp, const Traversal &tr, const std::vector<Oct> &nodes, int T,
-                             int max_terms, PointHost &out);
+// up, so every hanging point is a row.  Tiles of T elements, with at most
+// max_terms ends of rows.
+PtFit build_points_conforming(const MeshParams &mp, const Traversal &tr, const std::vector<Oct> &nodes, int T,
+                              int max_terms, PointHost &out);
 
 }  // namespace dkt
