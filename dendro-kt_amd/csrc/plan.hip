@@ -928,13 +928,19 @@ size_t size_points(dkt_plan *pl, const PointHost &o) {
 }
 
 // Leaves per tile: the requested size, else kPointTile, halved until the tiles fit
-// the layout and their LDS footprint (FP64) the limit.
+// the layout and their LDS footprint (FP64) the limit, and once where tiles end
+// at their readers, as on unbalanced trees: then a part of each workgroup idles,
+// and more of them wait for a chain of replays.  us for one FP64 column with 256 and
+// 128 (and 64) leaves, with the mean of the 256: 105 leaves, 2D, 539k in all, 29.0 and
+// 23.0 (21.9); 117, 3D, 1.56M, 84.0 and 72.5 (75.3); 155, 3D, 3.3M, 136 and 112; 178, 3D,
+// 399k, 24.9 and 22.4; 232, 2D, 491k, 15.8 and 15.2; balanced: 254, 3D, 117k, 13.7 and
+// 13.3; 250, 3D, 1.2M, 33.5 and 34.6; 256, 3D, 456k, 17.0 and 19.2.
 void build_points(dkt_plan *pl, const MeshParams &mp, const Traversal &tr, int requested) {
   int T = requested ? requested : kPointTile;
   while (true) {
     PointHost o;
-    if (build_points_reference(mp, tr, pl->N, T, std::max(1, T / pl->npe), o) == PtFit::yes &&
-        size_points(pl, o) <= kLdsLimit)
+    const int min_leaves = !requested && T == kPointTile ? kPointTile * 15 / 16 : 0;
+    if (build_points_reference(mp, tr, pl->N, T, min_leaves, o) == PtFit::yes && size_points(pl, o) <= kLdsLimit)
       return upload_points(pl, o, T);
     if (requested || T <= 64) throw std::runtime_error("tile does not fit in LDS");
     T /= 2;

@@ -417,7 +417,7 @@ size_t PointHost::bytes() const {
   return tiles.size() * sizeof(PtTile) + snode.size() * 8 + lloc.size() * 2 + (laux.size() + blocks.size()) * 4;
 }
 
-PtFit build_points_reference(const MeshParams &mp, const Traversal &tr, size_t N, int T, int n_groups, PointHost &out) {
+PtFit build_points_reference(const MeshParams &mp, const Traversal &tr, size_t N, int &T, int min_leaves, PointHost &out) {
   const int dim = mp.dim, npe = tr.nPe;
   const size_t L = tr.leaves.size();
   StaleBuffer sb(mp, tr);
@@ -455,25 +455,30 @@ PtFit build_points_reference(const MeshParams &mp, const Traversal &tr, size_t N
     for (uint32_t m = missing; m; m &= m - 1) n |= need[(size_t)c * npe + __builtin_ctz(m)];
     return n;
   };
+  // What the tile bounds depend on, per leaf.
+  enum { kHangs = 1, kReads = 2, kSibling = 4 };  // kSibling: the leaf before hangs, too, and has the same parent
+  std::vector<uint8_t> leaf(L);
+  constexpr size_t kLeaves = 2048;  // per unit of work
+  struct None {};
+  for_tiles<None>((L + kLeaves - 1) / kLeaves, [&](size_t u, None &) {
+    for (size_t e = u * kLeaves; e < std::min(L, (u + 1) * kLeaves); e++) {
+      if (tr.hang_of[e] < 0) continue;
+      uint32_t m, a;
+      masks(e, &m, &a);
+      leaf[e] = kHangs | ((needed(tr.child[e], m) & a) ? kReads : 0);
+      if (e > 0 && tr.hang_of[e - 1] >= 0 && same_oct(parent_of(e), parent_of(e - 1))) leaf[e] |= kSibling;
+    }
+  });
   // Tiles: runs of at most T leaves, kMaxTileReaders readers and T / 4 sibling
   // groups (a group: consecutive hanging leaves of one parent, cut at 64 leaves).
-  std::vector<size_t> bounds{0};
-  {
+  std::vector<size_t> bounds;
+  auto cut_tiles = [&]() {
+    bounds.assign(1, 0);
     const int max_groups = std::max(1, T / 4);
     int nrd = 0, ngrp = 0;
-    bool prev_hang = false;
-    Oct prev_par{};
     for (size_t e = 0; e < L; e++) {
-      bool reader = false, new_group = false;
-      Oct par{};
-      const bool hang = tr.hang_of[e] >= 0;
-      if (hang) {
-        uint32_t m, a;
-        masks(e, &m, &a);
-        reader = (needed(tr.child[e], m) & a) != 0;
-        par = parent_of(e);
-        new_group = !(prev_hang && same_oct(par, prev_par) && (e - bounds.back()) % 64 != 0);
-      }
+      const bool hang = leaf[e] & kHangs, reader = leaf[e] & kReads;
+      bool new_group = hang && !((leaf[e] & kSibling) && (e - bounds.back()) % 64 != 0);
       if (e - bounds.back() == (size_t)T || (reader && nrd == kMaxTileReaders) || (new_group && ngrp == max_groups)) {
         bounds.push_back(e);
         nrd = 0;
@@ -482,11 +487,15 @@ PtFit build_points_reference(const MeshParams &mp, const Traversal &tr, size_t N
       }
       nrd += reader ? 1 : 0;
       ngrp += new_group ? 1 : 0;
-      prev_hang = hang;
-      prev_par = par;
     }
     if (bounds.back() != L) bounds.push_back(L);
+  };
+  cut_tiles();
+  if (bounds.size() > 2 && L < (size_t)min_leaves * (bounds.size() - 2)) {
+    T /= 2;
+    cut_tiles();
   }
+  const int n_groups = std::max(1, T / npe);  // replay blocks per tile, a lane group each
   const size_t ntiles = bounds.size() - 1;
   PointHost o;
   o.lloc.resize(L * (size_t)npe);

@@ -94,9 +94,9 @@ struct PointHost {
 // fewer leaves per tile, or with none.
 enum class PtFit { yes, smaller, none };
 
-// Reference semantics over the flattened traversal, tiles of at most T leaves;
-// n_groups: replay blocks per tile.
-PtFit build_points_reference(const MeshParams &mp, const Traversal &tr, size_t N, int T, int n_groups, PointHost &out);
+// Reference semantics over the flattened traversal, tiles of at most T leaves.  T is
+// halved where the tiles (the last one aside) hold fewer than min_leaves on average.
+PtFit build_points_reference(const MeshParams &mp, const Traversal &tr, size_t N, int &T, int min_leaves, PointHost &out);
 
 // Conforming operator (sum_e C_e^T K_e C_e, build_conforming): a rank that is no
 // node takes its parent cell's interpolant, whose corners do the same one level

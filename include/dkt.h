@@ -55,7 +55,7 @@ extern "C" {
 /* Leaves per tile of the tiled path: flags |= log2(leaves) << DKT_PLAN_TILE_SHIFT
  * with leaves in {64, 128, 256}; 0 = 256 for p = 1 in 2D and 3D, else 128,
  * halved while the LDS footprint does not fit.  Tiles also end early at 32
- * stale-buffer readers. */
+ * stale-buffer readers; where that leaves fewer than 240 of the 256, 0 = 128. */
 #define DKT_PLAN_TILE_SHIFT 8
 
 typedef struct dkt_octs dkt_octs; /* host list of cells/points */
