@@ -247,20 +247,31 @@ __device__ __forceinline__ void tile_body(const TileArgs &A, int item, const T *
   // Node gathers in batches of kSB per work-item, all loads issued before use
   // and unconditionally, entries past the tile's nodes as its last node's (a
   // load inside a per-entry branch is waited for there; 4D, 2M points, FP32: 611
-  // us with branches, 597 so).
+  // us with branches, 597 so).  FP64 p = 1 keeps the branches, whose lanes past the
+  // nodes load nothing (4D, 43,726 elements: 28.0 us, 28.7 without; 225k 40.7 and
+  // 41.5; 2M points 968.4 and 969.2).
+  constexpr bool kGuard = P == 1 && sizeof(T) == 8;
+  auto node = [&](int j) -> int {
+    if constexpr (kGuard) return j < th.nnode ? nodes[j] : -1;
+    else return nodes[min(j, th.nnode - 1)];
+  };
+  auto value = [&](int g) -> T {
+    if constexpr (kGuard) return g >= 0 ? x[(size_t)g * A.ld] : T(0);
+    else return x[(size_t)g * A.ld];
+  };
   for (int j0 = tid; j0 < th.nnode; j0 += kSB * nthr) {
     int g[kSB];
 #pragma unroll
-    for (int b = 0; b < kSB; b++) g[b] = nodes[min(j0 + b * nthr, th.nnode - 1)];
+    for (int b = 0; b < kSB; b++) g[b] = node(j0 + b * nthr);
     T xv[kSB];
 #pragma unroll
-    for (int b = 0; b < kSB; b++) xv[b] = x[(size_t)g[b] * A.ld];
+    for (int b = 0; b < kSB; b++) xv[b] = value(g[b]);
     uint32_t d[kSB];
 #pragma unroll
     for (int b = 0; b < kSB; b++) d[b] = 0u;
     if (A.dir_in)
 #pragma unroll
-      for (int b = 0; b < kSB; b++) d[b] = A.dir_in[g[b]];
+      for (int b = 0; b < kSB; b++) d[b] = A.dir_in[kGuard ? max(g[b], 0) : g[b]];
 #pragma unroll
     for (int b = 0; b < kSB; b++)
       if (j0 + b * nthr < th.nnode) x_loc[j0 + b * nthr] = d[b] ? T(0) : xv[b];
