@@ -16,7 +16,7 @@
 //      interpolated in registers, IKD_Parent2Child, FEM/include/refel.h:214-240,
 //      or the replayed buffer for readers) and applies
 //      v = 2^(-level*hp) K_ref u (p = 1: in the Walsh-Hadamard basis that
-//      diagonalises K_ref; p = 2: dense, K_ref staged in LDS);
+//      diagonalises K_ref; p = 2: sum-factorised, one axis at a time);
 //   5. direct outputs are added into the LDS accumulator y_loc in nPe phases,
 //      one per rank (two disjoint leaves never share a node at the same rank,
 //      so a phase has no write conflicts);
