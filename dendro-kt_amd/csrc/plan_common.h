@@ -447,6 +447,33 @@ struct RankPhases {
         for (; k < w; k++) r[ph][k] = -1;
       }
   }
+  // Axes on which a rank is a midpoint, as a bit mask.
+  static constexpr int mids(int rank) {
+    int S = 0;
+    for (int d = 0; d < DIM; d++, rank /= 3) S |= (rank % 3 == 1) << d;
+    return S;
+  }
+  // Every rank once, and a phase's ranks of different S with equally many axes (the
+  // body rank aside).
+  constexpr bool sound() const {
+    constexpr int npe = DIM == 2 ? 9 : 27;
+    int seen[npe] = {};
+    for (int ph = 0; ph < n; ph++)
+      for (int k = 0; k < w; k++) {
+        const int a = r[ph][k];
+        if (a < 0) continue;
+        if (a >= npe || seen[a]++) return false;
+        for (int l = 0; l < k; l++) {
+          const int b = r[ph][l];
+          if (b < 0 || mids(a) == mids(b)) return false;
+          if (a != npe / 2 && b != npe / 2 && __builtin_popcount(mids(a)) != __builtin_popcount(mids(b))) return false;
+        }
+      }
+    for (int a = 0; a < npe; a++)
+      if (!seen[a]) return false;
+    return true;
+  }
 };
+static_assert(RankPhases<2>().sound() && RankPhases<3>().sound(), "ranks of a phase must not meet");
 
 }  // namespace dkt
