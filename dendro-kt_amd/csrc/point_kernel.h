@@ -2,8 +2,8 @@
 // column per workgroup, one leaf per work-item.
 //
 // The reference interpolates and transposes per leaf (FEM/include/matvec.h:
-// 403-522).  The 128 leaves of a 3D tile miss 350 ranks but only 114 different
-// positions, so here that work is done once per position:
+// 403-522).  128 leaves of a 3D sphere tree miss 340 ranks but only 112 different
+// positions (256: 680 and 210), so here that work is done once per position:
 //   1. stage the tile's nodes from x;
 //   2. rows: each hanging point is the mean of two earlier points, level by
 //      level; stale-buffer readers' points come from the replay (replay());
@@ -338,33 +338,37 @@ __device__ __forceinline__ void point_body(const PtArgs &A, int item, const T *_
   if (nlev < 2) __syncthreads();
   // Onto the nodes: first every quad's sum, in the quad's place (a node's list is
   // up to ten times the mean: dealt out by quad, no lane waits for another's
-  // list), then each node adds its quads up.
-  auto quad = [&](int i) -> T & { return *reinterpret_cast<T *>(quads + i); };
+  // list), then each node adds its quads up.  In FP64 for FP32 too, at no cost in
+  // time (24.8 and 24.7 us at 1.33M elements): a leaf's correction cancels its part of
+  // these sums, and summed in FP32 the matvec's error was 1 to 2 % (stiffness) and up to
+  // 14 % (mass) above that of interpolating per leaf; so it is the same.
+  auto quad = [&](int i) -> double & { return *reinterpret_cast<double *>(quads + i); };
   for (int i = tid; i < th.nquad; i += nthr) {
     const uint64_t w = quads[i];
-    quad(i) = (P[w & 0xFFFFu] + P[(w >> 16) & 0xFFFFu]) + (P[(w >> 32) & 0xFFFFu] + P[w >> 48]);
+    quad(i) = ((double)P[w & 0xFFFFu] + (double)P[(w >> 16) & 0xFFFFu]) +
+              ((double)P[(w >> 32) & 0xFFFFu] + (double)P[w >> 48]);
   }
   __syncthreads();
   // 6. Write-out.
   for (int j = tid, b = 0; j < nn; j += nthr, b++) {
     const int o = b == 0 ? o0[0] : b == 1 ? o0[1] : (int)block_a[nn + j];
     const bool zero = A.dir_out && A.dir_out[o >= 0 ? o : 0];
-    T acc = T(0);
+    double acc = 0.0;
     for (int s = 0; s < th.nqs; s++) {
       const uint4 st = steps4[s];
       if (j >= (int)(st.x >> 16)) break;  // steps cover ever fewer nodes
       const uint32_t sw[4] = {st.x, st.y, st.z, st.w};
-      T v[4];
+      double v[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const bool in = j < (int)(sw[i] >> 16);
         v[i] = quad(in ? (int)(sw[i] & 0xFFFFu) + j : 0);
-        v[i] = in ? v[i] : T(0);
+        v[i] = in ? v[i] : 0.0;
       }
       acc += (v[0] + v[1]) + (v[2] + v[3]);
     }
     if (o == INT32_MIN) continue;
-    const T r = fma(T(0.5), acc, P[j]);
+    const T r = (T)fma(0.5, acc, (double)P[j]);
     if (o >= 0)
       y[(size_t)o * A.ld + q] = zero ? T(0) : r;
     else
