@@ -582,7 +582,7 @@ class Batch:
         _chk(load().dkt_batch_run(self.h, ctypes.c_void_p(s)))
 
     def status(self):
-        """1 when a persistent launch's fix-up gave up waiting (results invalid), else 0."""
+        """0: no launch of a batch waits on another."""
         err = ctypes.c_int(0)
         _chk(load().dkt_batch_status(self.h, ctypes.byref(err)))
         return err.value

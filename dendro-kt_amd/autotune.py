@@ -3,9 +3,10 @@ counterpart in the reference).
 
 The tiled kernel's tile size trades LDS footprint (occupancy) against shared
 nodes between tiles.  With several right-hand sides a second choice appears:
-how many columns one launch carries.  More columns read the plan's maps once
-for all of them; fewer columns run kernels with fewer registers and more
-waves per SIMD (one column runs the single-column kernels).  ``autotune``
+how many columns one record of a launch carries.  Every column is a workgroup of
+its own; those of one record run next to each other and share the plan's maps and
+the lines of node-major vectors in L2, while single-column records run the kernels
+without a column index.  ``autotune``
 builds the plan of a sample mesh with each candidate tile size, times the
 FP64 and FP32 matvecs with HIP events on the launch stream (with nrhs > 1 as
 a one-plan batch for each candidate column count), and returns the fastest
@@ -30,7 +31,7 @@ def _column_candidates(nrhs):
     while c < nrhs:
         out.append(c)
         c *= 2
-    return tuple(out) + (0,)  # 0: as many as fit in LDS
+    return tuple(out) + (0,)  # 0: all of them
 
 
 def size_class(n_elements):

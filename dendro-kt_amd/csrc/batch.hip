@@ -3,13 +3,13 @@
 //
 // Plans of the same (dim, p) run as one launch: workgroup b finds its record
 // by a binary search over the records' tile offsets and runs that tile with
-// the record's maps and vectors (a device table of BatchPlan records, one per
-// plan and chunk of right-hand sides that fits the tiles' LDS, each chunk with
-// partial slots of its own), followed by one batched fix-up launch.  With
-// DKT_BATCH_GRAPH the two launches of every (dim, p) group are captured once
-// into a hipGraph and replayed.  Each plan's
-// result is bitwise the same as its own dkt_plan_matvec: the tile work and
-// the fix-up order are the plan's.
+// the record's maps and vectors (a device table with one record per plan and
+// chunk of right-hand sides, each with partial slots of its own; a chunk's
+// columns are workgroups of their own), and one fix-up launch sums the shared
+// nodes of all groups.  With DKT_BATCH_GRAPH the launches are captured once into a
+// hipGraph and replayed.  Each plan's result is bitwise the same as its own
+// dkt_plan_matvec: the tile work and the fix-up order are the plan's, whatever
+// the work-items of the launch.
 #include <algorithm>
 #include <map>
 #include <memory>
@@ -588,8 +588,8 @@ extern "C" int dkt_batch_create(dkt_plan *const *plans, int nplans, int dtype, i
     auto b = std::make_unique<dkt_batch>();
     if (flags & DKT_BATCH_PERSISTENT)
       throw std::invalid_argument(
-          "DKT_BATCH_PERSISTENT is switched off: its launch did not finish on the device and the cause is not "
-          "found; use the per-(dim, p) launches (with DKT_BATCH_GRAPH for a replayed graph)");
+          "DKT_BATCH_PERSISTENT is reserved: its kernel did not finish on the device and was removed; use the "
+          "per-(dim, p) launches (with DKT_BATCH_GRAPH for a replayed graph)");
     for (const auto &kv : by_kind_of(plans, nplans)) {
       std::vector<dkt_plan *> pls;
       std::vector<const void *> xs;

@@ -9,9 +9,12 @@
 // of kCgThreads work-items, fixed tree order): every block that needs alpha or
 // beta re-reduces the same partials in the same order, so all blocks agree
 // bit for bit and the solve is reproducible run to run.  Convergence raises a
-// device flag; the kernels of iterations queued after it (matvec included)
-// return at once, and the host only checks the flag every kCgChunk
-// iterations.
+// device flag, which the host only checks every kCgChunk iterations: the matvecs
+// queued after it return at once, the vector kernels read their first batch (the
+// loads do not wait for the flag) and write nothing.  In a batch a solve that has
+// stopped so costs its blocks' reads until the step ends; no batch was found to lose by
+// it (eight solves of up to 600k elements of which one, four or all run on: 0.80 to
+// 0.89 of the time with the tests first, the matvecs' gain by point tiles included).
 //
 // Mixed precision, DKT_CG_MIXED_RELIABLE: CG with reliable updates.  The iteration
 // runs with FP32 vectors and matvecs (FP32 accumulation inside the matvec) and

@@ -134,7 +134,7 @@ __device__ __forceinline__ void conf_tile_body(const ConfArgs &A, int item, cons
   // after its node ids, not kCB.  The values are loaded before the Dirichlet
   // flags, and everything unconditionally, entries past the tile's nodes as its
   // last node's: a load inside a per-entry branch is waited for there.
-  // The kernel is bound by these round trips (73 % of its wave time were
+  // The kernel is bound by these round trips (65 % of its wave time are
   // waits), so p = 2 in 3D, with 5 to 8 nodes a work-item, takes 8 at a time, and the
   // first rows' terms, the segments and the output slots are loaded a phase
   // early: 218 to 208 us on the 8.9M-node mesh in FP64, 172 to 163 in FP32.

@@ -948,9 +948,10 @@ void build_points(dkt_plan *pl, const MeshParams &mp, const Traversal &tr, int r
 }
 
 // The same for the conforming operator, tiles of T elements or fewer (1.33M
-// elements in 3D: FP64 36.5 -> 27.8 us, FP32 33.5 -> 23.4, eight FP64 columns 351
-// -> 207; captured 4D space-time matrices, 31k elements: 17.6 -> 13 us).  False: the
-// mesh does not fit point tiles of 64 elements, and takes conf_kernel.h's.
+// elements in 3D: FP64 35.5 -> 27.0 us, FP32 33.9 -> 24.1, eight FP64 columns 354
+// -> 211; captured 4D space-time matrices, 31k elements: 17.6 -> 13 us).  False: the
+// mesh does not fit point tiles of 64 elements (mostly: a chain of more than 11 row
+// levels), and takes conf_kernel.h's.
 bool build_conf_points(dkt_plan *pl, const MeshParams &mp, const Traversal &tr, const NodeSet &ns, int T) {
   for (; T >= 64; T /= 2) {
     PointHost o;

@@ -22,15 +22,16 @@ constexpr int kTileThreads = 256;
 constexpr int kDefaultTile = 128;
 // Reference-semantics plans on point tiles (point_kernel.h), the others on
 // tile_kernel.h.  p = 1 in 2D and 3D: the tiles share hanging positions and pass
-// few stale-buffer readers (FP64, 1.33M elements in 3D: 28 us against 41, eight
-// columns 140 against 461).  In 4D two thirds of a tile's rows come with a replay
+// few stale-buffer readers (FP64, 1.33M elements in 3D: 28 us against 40, eight
+// columns 214 against 559).  In 4D two thirds of a tile's rows come with a replay
 // of the stale buffer either way, and FP32 is faster on tile_kernel (15.3M
 // elements: FP64 852 us against 890, FP32 582 against 530).  p = 2 has no mean rows.
 constexpr bool point_tiles(int dim, int order) { return order == 1 && dim <= 3; }
-// Leaves per point tile, the fastest of 64, 128 and 256 (28.2, 28.0 and 27.3 us on
-// the 3D mesh above, eight columns 173, 148 and 140): larger tiles share more
+// Leaves per point tile, the fastest of 64, 128 and 256 (30.5, 28.9 and 28.0 us on
+// the 3D mesh above, eight columns 304, 237 and 216): larger tiles share more
 // points, and no leaf waits longer, since a barrier'd step is one round trip to
-// LDS whatever its width.
+// LDS whatever its width.  Where readers end the tiles early, 128 (build_points in
+// plan.hip).
 constexpr int kPointTile = 256;
 constexpr int kMaxConfTerms = 2048;  // constraint terms per conforming tile
 constexpr int kMaxConfVirt = 1024;   // hanging points per conforming tile

@@ -303,22 +303,17 @@ int dkt_cg_engine_destroy(dkt_cg_engine *engine);
  * each with its own device vectors x[k], y[k] of [N_k][nrhs] (dtype 0 f64,
  * 1 f32), plus one fix-up launch for the shared nodes of every plan.  flags
  * DKT_BATCH_GRAPH: the launches are captured into a hipGraph on the first
- * dkt_batch_run (the (dim, p) launches on parallel branches, joined before the
- * fix-up) and replayed after (the stream must not be the default stream;
- * the branches use streams of default priority).  Plans and vectors are bound at
+ * dkt_batch_run (the (dim, p) launches on parallel branches, the heaviest first,
+ * joined before the fix-up; large FP32 batches on one stream) and replayed after
+ * (the stream must not be the default stream; the branches use streams of default
+ * priority).  Plans and vectors are bound at
  * creation and must outlive the batch.  Every y[k] equals dkt_plan_matvec of
  * plan k bit for bit.  No counterpart in the reference (one fem::matvec per
  * call, FEM/include/matvec.h:231-240). */
 typedef struct dkt_batch dkt_batch;
 #define DKT_BATCH_GRAPH 1
-/* DKT_BATCH_PERSISTENT: one persistent launch per run for the whole batch,
- * any mix of (dim, p): the tiles of every plan (work claimed from eight
- * SFC-contiguous queues, one per XCD) and then the fix-up of their shared
- * nodes, each fix-up block waiting on its plan's tile-completion counter; the
- * kernel resets its counters on exit, so with DKT_BATCH_GRAPH a replay is one
- * graph node.  Tiled reference-semantics plans only.  Switched off:
- * dkt_batch_create refuses the flag (its launch did not finish on the device
- * and the cause is not found). */
+/* Reserved: dkt_batch_create refuses the flag.  It was one persistent launch for a
+ * whole batch; its kernel did not finish on the device and has been removed. */
 #define DKT_BATCH_PERSISTENT 2
 /* Columns per tile record for nrhs > 1: flags |= (log2(columns) + 1) <<
  * DKT_BATCH_COLUMNS_SHIFT with columns in {1, 2, 4, ..., 64}; 0 = all of
@@ -337,9 +332,8 @@ typedef struct dkt_batch dkt_batch;
 int dkt_batch_create(dkt_plan *const *plans, int nplans, int dtype, int nrhs, const void *const *x, void *const *y,
                      int masked, int flags, dkt_batch **out);
 int dkt_batch_run(dkt_batch *batch, void *stream);
-/* Persistent batches: *err = 1 when a fix-up block gave up waiting for its
- * plan's tiles (a bounded spin; the results of that run are not valid), else 0.
- * Synchronizes with the device. */
+/* *err = 0: no launch of a batch waits on another (the call stays for callers of
+ * the removed persistent launch). */
 int dkt_batch_status(dkt_batch *batch, int *err);
 int dkt_batch_destroy(dkt_batch *batch);
 
