@@ -15,9 +15,7 @@
 // dof-interleaved layout, include/oda.h:296-322).
 #include <algorithm>
 #include <atomic>
-#include <exception>
 #include <mutex>
-#include <thread>
 #include <array>
 #include <cmath>
 #include <cstring>
@@ -34,6 +32,7 @@
 #include "tile_kernel.h"
 #include "conf_kernel.h"
 #include "point_kernel.h"
+#include "threads.h"
 
 namespace dkt {
 const MeshParams &da_params(const dkt_da *da);
@@ -740,12 +739,8 @@ TiledHost build_tiled_host(const MeshParams &mp, const Traversal &tr, size_t N, 
     for (const auto &e : ent) to.hent.push_back(e.second);
   };
   {
-    const unsigned hw = std::thread::hardware_concurrency();
-    const int nthreads = (int)std::max(1u, std::min(16u, hw ? hw : 1u));
     std::atomic<size_t> next{0};
-    std::exception_ptr err;
-    std::mutex err_mu;
-    auto worker = [&]() {
+    on_threads(host_threads(), [&]() {
       try {
         LocalMap lm;
         std::unordered_map<uint64_t, Combo> memo;
@@ -756,16 +751,10 @@ TiledHost build_tiled_host(const MeshParams &mp, const Traversal &tr, size_t N, 
           for (size_t t = t0; t < std::min(ntiles, t0 + 16); t++) build_tile(t, outs[t], lm, memo);
         }
       } catch (...) {
-        std::lock_guard<std::mutex> g(err_mu);
-        if (!err) err = std::current_exception();
         next.store(ntiles);
+        throw;
       }
-    };
-    std::vector<std::thread> pool;
-    for (int i = 1; i < nthreads; i++) pool.emplace_back(worker);
-    worker();
-    for (auto &th : pool) th.join();
-    if (err) std::rethrow_exception(err);
+    });
   }
   // Concatenation in tile order; shared nodes get their partial slots in tile order.
   double s_rd = 0, m_rd = 0, s_cr = 0, m_cr = 0, s_gr = 0, s_nn = 0, s_cone = 0, n_cone = 0;
@@ -1065,13 +1054,7 @@ void build_conf_tiled(dkt_plan *pl, const MeshParams &mp, const Traversal &tr, i
         }
       }
     };
-    {
-      const unsigned hw = std::thread::hardware_concurrency();
-      std::vector<std::thread> pool;
-      for (unsigned i = 1; i < std::max(1u, std::min(16u, hw ? hw : 1u)); i++) pool.emplace_back(scan);
-      scan();
-      for (auto &th : pool) th.join();
-    }
+    on_threads(host_threads(), scan);
     for (const auto &d : part) wbits.insert(wbits.end(), d.begin(), d.end());
     std::sort(wbits.begin(), wbits.end());
     wbits.erase(std::unique(wbits.begin(), wbits.end()), wbits.end());
@@ -1166,12 +1149,8 @@ void build_conf_tiled(dkt_plan *pl, const MeshParams &mp, const Traversal &tr, i
     }
   };
   {
-    const unsigned hw = std::thread::hardware_concurrency();
-    const int nthreads = (int)std::max(1u, std::min(16u, hw ? hw : 1u));
     std::atomic<size_t> next{0};
-    std::exception_ptr err;
-    std::mutex err_mu;
-    auto worker = [&]() {
+    on_threads(host_threads(), [&]() {
       try {
         Scratch sc;
         while (true) {
@@ -1180,16 +1159,10 @@ void build_conf_tiled(dkt_plan *pl, const MeshParams &mp, const Traversal &tr, i
           for (size_t t = t0; t < std::min(ntiles, t0 + 16); t++) build_tile(t, outs[t], sc);
         }
       } catch (...) {
-        std::lock_guard<std::mutex> g(err_mu);
-        if (!err) err = std::current_exception();
         next.store(ntiles);
+        throw;
       }
-    };
-    std::vector<std::thread> pool;
-    for (int i = 1; i < nthreads; i++) pool.emplace_back(worker);
-    worker();
-    for (auto &th : pool) th.join();
-    if (err) std::rethrow_exception(err);
+    });
   }
   std::vector<ConfTileHdr> hdr(ntiles);
   std::vector<int32_t> tnodes;

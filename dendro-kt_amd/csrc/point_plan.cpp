@@ -23,10 +23,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <exception>
-#include <mutex>
 #include <stdexcept>
-#include <thread>
+
+#include "threads.h"
 
 namespace dkt {
 
@@ -274,12 +273,9 @@ void finish_tile(TileOut &to, PointSet &ps, const std::vector<uint16_t> &corr, R
 constexpr size_t kGrain = 6;
 template <typename Scratch, typename F>
 void for_tiles(size_t ntiles, F &&work) {
-  const unsigned hw = std::thread::hardware_concurrency();
-  const int nthreads = (int)std::min<size_t>(std::max(1u, std::min(16u, hw ? hw : 1u)), (ntiles + kGrain - 1) / kGrain);
+  const int nthreads = (int)std::min<size_t>(host_threads(), (ntiles + kGrain - 1) / kGrain);
   std::atomic<size_t> next{0};
-  std::exception_ptr err;
-  std::mutex mu;
-  auto worker = [&]() {
+  on_threads(nthreads, [&]() {
     try {
       Scratch sc;
       while (true) {
@@ -288,16 +284,10 @@ void for_tiles(size_t ntiles, F &&work) {
         for (size_t t = t0; t < std::min(ntiles, t0 + kGrain); t++) work(t, sc);
       }
     } catch (...) {
-      std::lock_guard<std::mutex> g(mu);
-      if (!err) err = std::current_exception();
       next.store(ntiles);
+      throw;
     }
-  };
-  std::vector<std::thread> pool;
-  for (int i = 1; i < nthreads; i++) pool.emplace_back(worker);
-  worker();
-  for (auto &th : pool) th.join();
-  if (err) std::rethrow_exception(err);
+  });
 }
 
 // Partial slots of the nodes that several tiles write (consecutive per node,
